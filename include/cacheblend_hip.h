@@ -375,6 +375,22 @@ int cbk_blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int
                         float scale, int32_t dtype, void* out_dev, int64_t out_row_stride_elems,
                         cbk_stream_t stream);
 
+/*
+ * The same with device scratch: a launch whose row tiles do not fill the GPU
+ * then splits every tile's keys into ranges and merges their partial results
+ * (float32). workspace_bytes: at least what the _workspace_bytes function
+ * gives for the sizes on the current device (0: the launch takes one range);
+ * workspace_dev 256-byte aligned, NULL for one range whatever the sizes (as
+ * cbk_blend_attention). CBK_ERR_WORKSPACE if it is too small.
+ */
+size_t cbk_blend_attention_workspace_bytes(int64_t nq, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim,
+                                           int32_t dtype);
+int cbk_blend_attention_ws(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev, int64_t nq,
+                           const void* k_dev, int64_t k_row_stride_elems, const void* v_dev,
+                           int64_t v_row_stride_elems, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim,
+                           float scale, int32_t dtype, void* out_dev, int64_t out_row_stride_elems,
+                           void* workspace_dev, size_t workspace_bytes, cbk_stream_t stream);
+
 /* Workspace bytes cbk_sparse_q_scores needs: row statistics, a record per
  * 16-query tile, per-KV-head partial column sums and a dense copy of the
  * query rows (sized for head_dim 128): about nq * hq * 264 + nk * hkv * 4

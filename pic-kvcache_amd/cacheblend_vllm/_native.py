@@ -148,6 +148,12 @@ _SIGNATURES = {
         [c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.c_float,
          c_i32, c_vp, c_i64, c_vp],
     ),
+    "cbk_blend_attention_workspace_bytes": (ctypes.c_size_t, [c_i64, c_i64, c_i64, c_i64, c_i64, c_i32]),
+    "cbk_blend_attention_ws": (
+        ctypes.c_int,
+        [c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, ctypes.c_float,
+         c_i32, c_vp, c_i64, c_vp, ctypes.c_size_t, c_vp],
+    ),
     "cbk_rolling_hashes": (ctypes.c_int, [c_vp, c_i64, c_i64, c_vp]),
     "cbk_matcher_create": (ctypes.c_int, [c_i64, ctypes.POINTER(c_vp)]),
     "cbk_matcher_destroy": (ctypes.c_int, [c_vp]),

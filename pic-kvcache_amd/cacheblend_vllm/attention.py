@@ -53,11 +53,17 @@ def blend_attention(
     out = torch.empty((nq, hq, d), dtype=query.dtype, device=query.device)
     if nq == 0:
         return out
-    rc = _native.load().cbk_blend_attention(
+    lib = _native.load()
+    # partial results of the keys' ranges, from torch's allocator on every
+    # call: a captured graph then owns its own
+    dtype_code = _native.DTYPE_CODES[query.dtype]
+    nbytes = lib.cbk_blend_attention_workspace_bytes(nq, nk, hq, hkv, d, dtype_code)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
+    rc = lib.cbk_blend_attention_ws(
         query.data_ptr(), query.stride(0), pos.data_ptr(), nq,
         key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0), nk, hq, hkv, d,
-        float(scale), _native.DTYPE_CODES[query.dtype], out.data_ptr(), out.stride(0),
-        _native.stream_handle(query.device),
+        float(scale), dtype_code, out.data_ptr(), out.stride(0),
+        _native.ptr(ws), nbytes, _native.stream_handle(query.device),
     )
     _native.check(rc, "blend_attention")
     return out

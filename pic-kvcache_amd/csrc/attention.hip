@@ -33,14 +33,14 @@
 // element k%8, B[k][j] in lane j+16*(k/8); D[i][j] in lane j+16*(i/4),
 // register i%4.
 //
-// float32 inputs take an exact float32 path (one wave per (query, head)).
+// float32 inputs: attention_f32.hip.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
 #include <cmath>
 #include <type_traits>
 
-#include "cbk_common.hpp"
+#include "attention_split.hpp"
 
 namespace cbk {
 namespace {
@@ -689,75 +689,40 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   }
 }
 
-// float32: one wave per (query, head), exact float32 dots and accumulation,
-// two dims per lane (D <= 128).
-struct AttnArgsF32 {
-  const float* q;
-  const int64_t* pos;
-  const float* k;
-  const float* v;
-  float* out;
-  int64_t q_stride, k_stride, v_stride, out_stride;
-  uint32_t nq, nk, hq, hkv, group, d;
-  float scale;
-};
-
-__global__ __launch_bounds__(256) void attn_f32_kernel(const AttnArgsF32 a) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t job = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (job >= a.nq * a.hq) return;  // whole waves exit together
-  const uint32_t qi = job / a.hq, h = job % a.hq, kvh = h / a.group;
-  const float* q = a.q + int64_t(qi) * a.q_stride + int64_t(h) * a.d;
-  const float q0 = lane < a.d ? q[lane] : 0.f;
-  const float q1 = lane + 64 < a.d ? q[lane + 64] : 0.f;
-  int64_t last = a.pos[qi];
-  if (last >= int64_t(a.nk)) last = int64_t(a.nk) - 1;
-  float m = kNegInf, l = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int64_t j = 0; j <= last; ++j) {
-    const float* kr = a.k + j * a.k_stride + int64_t(kvh) * a.d;
-    const float* vr = a.v + j * a.v_stride + int64_t(kvh) * a.d;
-    float dot = (lane < a.d ? q0 * kr[lane] : 0.f) + (lane + 64 < a.d ? q1 * kr[lane + 64] : 0.f);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
-    const float x = dot * a.scale;
-    const float mn = fmaxf(m, x);
-    const float alpha = expf(m - mn);
-    const float p = expf(x - mn);
-    l = l * alpha + p;
-    o0 = o0 * alpha + p * (lane < a.d ? vr[lane] : 0.f);
-    o1 = o1 * alpha + p * (lane + 64 < a.d ? vr[lane + 64] : 0.f);
-    m = mn;
-  }
-  float* out = a.out + int64_t(qi) * a.out_stride + int64_t(h) * a.d;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (lane < a.d) out[lane] = o0 * inv;
-  if (lane + 64 < a.d) out[lane + 64] = o1 * inv;
-}
-
 }  // namespace
 }  // namespace cbk
 
-extern "C" int cbk_blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev,
-                                   int64_t nq, const void* k_dev, int64_t k_row_stride_elems,
-                                   const void* v_dev, int64_t v_row_stride_elems, int64_t nk, int64_t hq,
-                                   int64_t hkv, int64_t head_dim, float scale, int32_t dtype, void* out_dev,
-                                   int64_t out_row_stride_elems, cbk_stream_t stream) {
-  using namespace cbk;
-  clear_error();
+namespace cbk {
+namespace {
+
+// Key ranges of a launch (attn_splits) for inputs that passed the checks.
+uint32_t launch_splits(int64_t nq, int64_t nk, int64_t hq, int64_t hkv, int32_t dtype) {
+  if (dtype != CBK_DTYPE_F32) return 1;
+  const uint64_t nrows = uint64_t(nq) * uint64_t(hq / hkv);
+  const uint64_t groups = (nrows + kAttnF32Rows - 1) / kAttnF32Rows * uint64_t(hkv);
+  return attn_splits(groups, kAttnF32PerCu, nk);
+}
+
+int check_sizes(int64_t nq, int64_t nk, int64_t hq, int64_t hkv) {
   CBK_REQUIRE(nq >= 0 && nq < (int64_t(1) << 26), "nq out of range");
-  if (nq == 0) return CBK_OK;
-  CBK_REQUIRE(q_dev && q_pos_dev && k_dev && v_dev && out_dev, "NULL pointer");
   CBK_REQUIRE(nk > 0 && nk < (int64_t(1) << 31), "nk out of range");
   CBK_REQUIRE(hq > 0 && hkv > 0 && hq % hkv == 0, "query heads must be divisible by KV heads");
   CBK_REQUIRE(nq * hq < (int64_t(1) << 31), "nq * hq too large");
+  return CBK_OK;
+}
+
+int blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev, int64_t nq,
+                    const void* k_dev, int64_t k_row_stride_elems, const void* v_dev, int64_t v_row_stride_elems,
+                    int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim, float scale, int32_t dtype, void* out_dev,
+                    int64_t out_row_stride_elems, const AttnParts& parts, hipStream_t s) {
+  CBK_REQUIRE(q_dev && q_pos_dev && k_dev && v_dev && out_dev, "NULL pointer");
   CBK_REQUIRE(q_row_stride_elems >= hq * head_dim && out_row_stride_elems >= hq * head_dim &&
                   k_row_stride_elems >= hkv * head_dim && v_row_stride_elems >= hkv * head_dim,
               "row stride smaller than a row");
   CBK_REQUIRE(std::isfinite(scale), "scale must be finite");
-  const hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == CBK_DTYPE_F32) {
     CBK_REQUIRE(head_dim > 0 && head_dim <= 128, "float32 path needs head_dim <= 128");
-    AttnArgsF32 a;
+    AttnF32Args a;
     a.q = static_cast<const float*>(q_dev);
     a.pos = q_pos_dev;
     a.k = static_cast<const float*>(k_dev);
@@ -774,9 +739,10 @@ extern "C" int cbk_blend_attention(const void* q_dev, int64_t q_row_stride_elems
     a.group = uint32_t(hq / hkv);
     a.d = uint32_t(head_dim);
     a.scale = scale;
-    const uint64_t jobs = uint64_t(nq) * uint64_t(hq);
-    hipLaunchKernelGGL(attn_f32_kernel, dim3(uint32_t((jobs + 3) / 4)), dim3(256), 0, s, a);
-    return launch_status("blend attention f32");
+    a.parts = parts;
+    if (int rc = launch_attn_f32(a, s)) return rc;
+    if (parts.splits == 1) return CBK_OK;
+    return launch_attn_merge(parts, a.nq, a.hq, a.d, q_pos_dev, out_dev, out_row_stride_elems, dtype, true, s);
   }
   CBK_REQUIRE(dtype == CBK_DTYPE_BF16 || dtype == CBK_DTYPE_F16, "dtype %d", int(dtype));
   CBK_REQUIRE(head_dim == 64 || head_dim == 128, "head_dim %lld: 64 or 128 supported", (long long)head_dim);
@@ -823,3 +789,51 @@ extern "C" int cbk_blend_attention(const void* q_dev, int64_t q_row_stride_elems
   }
   return launch_status("blend attention");
 }
+
+}  // namespace
+}  // namespace cbk
+
+extern "C" {
+
+size_t cbk_blend_attention_workspace_bytes(int64_t nq, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim,
+                                           int32_t dtype) {
+  using namespace cbk;
+  if (check_sizes(nq, nk, hq, hkv) || nq == 0 || head_dim <= 0 || head_dim > 128) return 0;
+  return attn_parts_bytes(launch_splits(nq, nk, hq, hkv, dtype), uint64_t(nq) * uint64_t(hq), head_dim);
+}
+
+int cbk_blend_attention_ws(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev, int64_t nq,
+                           const void* k_dev, int64_t k_row_stride_elems, const void* v_dev,
+                           int64_t v_row_stride_elems, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim,
+                           float scale, int32_t dtype, void* out_dev, int64_t out_row_stride_elems,
+                           void* workspace_dev, size_t workspace_bytes, cbk_stream_t stream) {
+  using namespace cbk;
+  clear_error();
+  if (int rc = check_sizes(nq, nq == 0 ? 1 : nk, nq == 0 ? 1 : hq, nq == 0 ? 1 : hkv)) return rc;
+  if (nq == 0) return CBK_OK;
+  // without a workspace one range: every tile's keys in one workgroup
+  uint32_t splits = 1;
+  const uint64_t rows = uint64_t(nq) * uint64_t(hq);
+  if (workspace_dev != nullptr) {
+    splits = launch_splits(nq, nk, hq, hkv, dtype);
+    if (workspace_bytes < attn_parts_bytes(splits, rows, head_dim))
+      return set_error(CBK_ERR_WORKSPACE, "attention workspace %zu < %zu bytes", workspace_bytes,
+                       attn_parts_bytes(splits, rows, head_dim));
+    CBK_REQUIRE((reinterpret_cast<uintptr_t>(workspace_dev) & 255) == 0, "workspace must be 256-byte aligned");
+  }
+  return blend_attention(q_dev, q_row_stride_elems, q_pos_dev, nq, k_dev, k_row_stride_elems, v_dev,
+                         v_row_stride_elems, nk, hq, hkv, head_dim, scale, dtype, out_dev, out_row_stride_elems,
+                         attn_parts(splits, rows, workspace_dev), static_cast<hipStream_t>(stream));
+}
+
+int cbk_blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev, int64_t nq,
+                        const void* k_dev, int64_t k_row_stride_elems, const void* v_dev,
+                        int64_t v_row_stride_elems, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim,
+                        float scale, int32_t dtype, void* out_dev, int64_t out_row_stride_elems,
+                        cbk_stream_t stream) {
+  return cbk_blend_attention_ws(q_dev, q_row_stride_elems, q_pos_dev, nq, k_dev, k_row_stride_elems, v_dev,
+                                v_row_stride_elems, nk, hq, hkv, head_dim, scale, dtype, out_dev,
+                                out_row_stride_elems, nullptr, 0, stream);
+}
+
+}  // extern "C"

@@ -25,6 +25,9 @@ void clear_error();
 // Returns CBK_OK, or CBK_ERR_LAUNCH with the HIP error of the last launch.
 int launch_status(const char* what);
 
+// Compute units of the current device (cached per device).
+int device_cus(int* cus);
+
 // ---------------------------------------------------------- fast divide
 // Unsigned 32-bit division by a runtime constant d >= 1 (Granlund-Montgomery
 // round-up method): q = (umulhi(n, m) + n) >> s, exact for every n < 2^32.

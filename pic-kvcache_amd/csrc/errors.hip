@@ -1,4 +1,6 @@
 // Error reporting shared by every entry point of libcacheblend_hip.so.
+#include <mutex>
+
 #include "cbk_common.hpp"
 
 namespace cbk {
@@ -22,6 +24,23 @@ int launch_status(const char* what) {
   if (err != hipSuccess) {
     return set_error(CBK_ERR_LAUNCH, "%s: %s", what, hipGetErrorString(err));
   }
+  return CBK_OK;
+}
+
+int device_cus(int* cus) {
+  static std::mutex mu;
+  static int cached[64] = {};
+  int dev = 0;
+  hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return set_error(CBK_ERR_LAUNCH, "hipGetDevice: %s", hipGetErrorString(err));
+  std::lock_guard<std::mutex> lock(mu);
+  if (dev >= 0 && dev < 64 && cached[dev] > 0) {
+    *cus = cached[dev];
+    return CBK_OK;
+  }
+  err = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (err != hipSuccess) return set_error(CBK_ERR_LAUNCH, "CU count: %s", hipGetErrorString(err));
+  if (dev >= 0 && dev < 64) cached[dev] = *cus;
   return CBK_OK;
 }
 

@@ -36,7 +36,6 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
-#include <mutex>
 #include <type_traits>
 
 #include "cbk_common.hpp"
@@ -977,24 +976,6 @@ __host__ SqLayout sq_layout(int64_t nq, int64_t nk, int64_t hq, int64_t hkv) {
   L.chunk_stats = (L.qdense + (uint64_t(L.nq_pad) * hq + 4 * kQTile) * kMaxHeadDim * 2 + 255) & ~uint64_t(255);
   L.bytes = (L.chunk_stats + uint64_t(kMaxRowChunks) * hq * L.nq_pad * 8 + 255) & ~uint64_t(255);
   return L;
-}
-
-// Compute units of the current device (cached per device).
-int device_cus(int* cus) {
-  static std::mutex mu;
-  static int cached[64] = {};
-  int dev = 0;
-  hipError_t err = hipGetDevice(&dev);
-  if (err != hipSuccess) return set_error(CBK_ERR_LAUNCH, "hipGetDevice: %s", hipGetErrorString(err));
-  std::lock_guard<std::mutex> lock(mu);
-  if (dev >= 0 && dev < 64 && cached[dev] > 0) {
-    *cus = cached[dev];
-    return CBK_OK;
-  }
-  err = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (err != hipSuccess) return set_error(CBK_ERR_LAUNCH, "CU count: %s", hipGetErrorString(err));
-  if (dev >= 0 && dev < 64) cached[dev] = *cus;
-  return CBK_OK;
 }
 
 // Key ranges per (query tile, kv head) in rowstats: tiles differ in work by

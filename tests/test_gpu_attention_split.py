@@ -1,0 +1,100 @@
+"""GPU parity of the attention kernels' row tiles, key blocks and key ranges,
+at the sizes where they end unevenly, against float64."""
+
+import numpy as np
+import pytest
+import torch
+
+from cacheblend_vllm import _native
+from cacheblend_vllm.attention import blend_attention
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def _f64(q, k, v, pos, scale):
+    """(outputs, sum_k p_k |v_k|, largest sum_i |q_i k_i|) in float64."""
+    nq, hq, d = q.shape
+    g = hq // k.shape[1]
+    out, mass, size = np.zeros((nq, hq, d)), np.zeros((nq, hq, d)), 0.0
+    visible = pos.numpy()[:, None] >= np.arange(k.shape[0])[None, :]
+    for h in range(hq):
+        qh, kh, vh = (t.double().numpy() for t in (q[:, h], k[:, h // g], v[:, h // g]))
+        x = np.where(visible, qh @ kh.T * scale, -np.inf)
+        e = np.exp(x - x.max(axis=1, keepdims=True, initial=-1e300))
+        p = e / np.maximum(e.sum(axis=1, keepdims=True), 1e-300)
+        out[:, h], mass[:, h] = p @ vh, p @ np.abs(vh)
+        size = max(size, float((np.abs(qh) @ np.abs(kh).T).max()))
+    return out, mass, size
+
+
+def _f32_bound(mass, size, d, nk, scale):
+    """What float32 can move an output by: a logit by (d + 3) roundings of at
+    most 2^-24 of its absolute terms, hence its probability by that factor (and
+    the sum it is divided by, once more), and each of the two sums over nk keys
+    and the exponential by at most (nk + 8) roundings."""
+    u = 2.0 ** -24
+    return (2 * np.expm1((d + 3) * u * size * scale) + 2 * (nk + 8) * u) * mass + 1e-30
+
+
+def _inputs(nq, nk, hq, hkv, d, dtype=torch.float32, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(n, h, d, generator=g).to(dtype) for n, h in ((nq, hq), (nk, hkv), (nk, hkv)))
+    pos = torch.randint(0, nk, (nq,), generator=g)
+    pos[-1] = nk - 1
+    return q, k, v, pos
+
+
+# rows of (query, group head) around the 64-row tile, keys around the 32-key
+# block, head sizes around the padded 64 and 128, and more ranges than a tile
+# with few keys has blocks
+@pytest.mark.parametrize("nq,nk,hq,hkv,d", [
+    (1, 1, 1, 1, 128), (1, 33, 2, 1, 64), (16, 32, 4, 1, 128), (63, 300, 2, 2, 64), (65, 257, 3, 1, 128),
+    (22, 1031, 6, 2, 100), (5, 4099, 8, 8, 128), (9, 700, 4, 2, 3), (40, 513, 4, 4, 66), (130, 2047, 16, 8, 128),
+])
+def test_f32_matches_float64(nq, nk, hq, hkv, d):
+    q, k, v, pos = _inputs(nq, nk, hq, hkv, d)
+    scale = d ** -0.5
+    got = blend_attention(q.to(DEV), k.to(DEV), v.to(DEV), pos.to(DEV), scale).cpu().numpy()
+    want, mass, size = _f64(q, k, v, pos, scale)
+    err = np.abs(got - want)
+    print(f"largest error / bound {(err / _f32_bound(mass, size, d, nk, scale)).max():.3f}", flush=True)
+    assert np.all(err <= _f32_bound(mass, size, d, nk, scale))
+
+
+def test_f32_unaligned_views_and_one_range():
+    # rows 4 bytes off a 16-byte boundary, and the entry without a workspace
+    nq, nk, hq, hkv, d = 37, 901, 4, 2, 64
+    q, k, v, pos = _inputs(nq, nk, hq, hkv, d, seed=1)
+    want, mass, size = _f64(q, k, v, pos, 0.125)
+    bound = _f32_bound(mass, size, d, nk, 0.125)
+
+    def off(t):
+        flat = torch.zeros(t.shape[0], t.shape[1] * d + 1)
+        flat[:, 1:] = t.reshape(t.shape[0], -1)
+        return flat.to(DEV)[:, 1:].unflatten(1, (t.shape[1], d))
+
+    got = blend_attention(off(q), off(k), off(v), pos.to(DEV), 0.125).cpu().numpy()
+    assert np.all(np.abs(got - want) <= bound)
+    dq, dk, dv, dp = (t.to(DEV) for t in (q, k, v, pos))
+    out = torch.empty_like(dq)
+    rc = _native.load().cbk_blend_attention(
+        dq.data_ptr(), hq * d, dp.data_ptr(), nq, dk.data_ptr(), hkv * d, dv.data_ptr(), hkv * d, nk, hq, hkv, d,
+        0.125, _native.DTYPE_CODES[torch.float32], out.data_ptr(), hq * d, _native.stream_handle(DEV))
+    _native.check(rc, "blend_attention")
+    assert np.all(np.abs(out.cpu().numpy() - want) <= bound)
+
+
+def test_f32_values_past_a_position_do_not_reach_its_row():
+    # keys and values past each position hold NaN and infinities; rows that
+    # see one have it in their result; a position below 0 sees nothing
+    nq, nk, hq, hkv, d = 20, 400, 2, 1, 64
+    q, k, v, _ = _inputs(nq, nk, hq, hkv, d, seed=2)
+    pos = torch.arange(nq) * 20 - 1
+    want, mass, size = _f64(q, k, v, pos.clamp(min=0), 0.125)
+    k[300], v[300], v[310, 0, 5], k[330] = float("nan"), float("inf"), float("nan"), float("inf")
+    got = blend_attention(q.to(DEV), k.to(DEV), v.to(DEV), pos.to(DEV), 0.125).cpu().numpy()
+    clean = (pos.numpy() < 300) & (pos.numpy() >= 0)
+    assert np.all(np.abs(got - want)[clean] <= _f32_bound(mass, size, d, nk, 0.125)[clean])
+    assert np.all(got[pos.numpy() < 0] == 0)
+    assert np.all(np.isnan(got[pos.numpy() >= 300]))
