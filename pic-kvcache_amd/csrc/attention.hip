@@ -27,7 +27,7 @@
 //                   row-major V block
 // software-pipelined: the step of block b issues S^T of block b+1 and P . V
 // of block b-1 beside the softmax of block b. K/V blocks stream through
-// rings of three LDS buffers by DMA (global_load_lds); the row tiles with the
+// rings of four LDS buffers by DMA (global_load_lds); the row tiles with the
 // latest positions (most keys) are scheduled first.
 // MFMA layout (checked on gfx950): 16x16x32 A[i][k] in lane i+16*(k/8)
 // element k%8, B[k][j] in lane j+16*(k/8); D[i][j] in lane j+16*(i/4),
@@ -62,7 +62,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // SIMD): 2.02-2.04 vs 2.12-2.15 ms per C3 layer.
 constexpr int kWaves = 4;
 constexpr int kRowTiles = 2;  // 16-row tiles per wave
-constexpr int kKeyBlock = 32;
+constexpr int kKeyBlock = kAttnKeyBlock;
+// Workgroups per CU that the key ranges aim at: as many as are resident.
+constexpr uint32_t per_cu(int64_t head_dim) { return head_dim == 64 ? 3 : 2; }
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kNegInf = -__builtin_inff();
@@ -77,6 +79,7 @@ struct AttnArgs {
   int64_t q_stride, k_stride, v_stride, out_stride;
   uint32_t nq, nk, hq, hkv, group, d;
   float scale;
+  AttnParts parts;
 };
 
 template <bool F16> struct Ops;
@@ -266,9 +269,10 @@ __device__ __forceinline__ void pv_block(const uint16_t* vs, const BlockOffsets<
   for (int t = 0; t < RT; ++t) ol[t] = O::mma32(pa[t], ones, ol[t]);
 }
 
-// K and V blocks of 32 keys stream through rings of three LDS buffers by DMA
+// K and V blocks of 32 keys stream through rings of four LDS buffers by DMA
 // (global_load_lds, explicit vmcnt waits, plain s_barrier; see the LDS DMA
-// helpers): K three blocks ahead of the step that reads it, V one.
+// helpers), requested three steps ahead of the one that reads them (two, with
+// rings of three: 0.5-1% slower, and six steps of code instead of four).
 template <bool F16, int D, int RT>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2))) void attn_kernel(
     const AttnArgs a) {
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   constexpr uint32_t P = D / 8;                      // 16-byte pieces per key row
   constexpr uint32_t kInsts = kKeyBlock * P / 64 / W; // requests per wave per block, each of K and V
   constexpr uint32_t kRowsPerInst = 64 / P;
-  constexpr int kBuffers = 3;
+  constexpr int kBuffers = 4;
   static_assert(kInsts >= 1 && W * 16 * D <= 2 * kBuffers * kKeyBlock * D, "wave count vs block and staging");
   // K blocks, then V blocks; the output staging reuses the whole region
   __shared__ __attribute__((aligned(16))) uint16_t kvbuf[2][kBuffers][kKeyBlock * D];
@@ -289,13 +293,16 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   // runtime value runs on the VALU), so what derives from them stays scalar
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t row = lane & 15, grp = lane >> 4;
-  // workgroup -> (row tile, kv head), the kv head fastest and the latest
-  // tiles (most keys) first: work is dispatched in decreasing order across
-  // all heads
+  // workgroup -> (row tile, key range, kv head), the kv head fastest and the
+  // latest tiles (most keys) first: work is dispatched in decreasing order
+  // across all heads
+  const uint32_t S = a.parts.splits;
   const uint32_t kvh = __builtin_amdgcn_readfirstlane(blockIdx.x % a.hkv);
+  const uint32_t rest = __builtin_amdgcn_readfirstlane(blockIdx.x / a.hkv);
+  const uint32_t split = __builtin_amdgcn_readfirstlane(rest % S);
   const uint32_t nrows = a.nq * a.group;
   const uint32_t ntiles = (nrows + kRows - 1) / kRows;
-  const uint32_t tile = __builtin_amdgcn_readfirstlane(ntiles - 1 - blockIdx.x / a.hkv);
+  const uint32_t tile = __builtin_amdgcn_readfirstlane(ntiles - 1 - rest / S);
   const uint32_t r_wave = tile * kRows + wave * 16 * RT;
 
   // this lane's rows (one per row tile): (query, head) and their Q fragments
@@ -333,9 +340,22 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
 #pragma unroll
   for (int w = 1; w < W; ++w) gm = max(gm, s_max[w]);
   const int32_t gmax = __builtin_amdgcn_readfirstlane(gm);
-  // blocks up to the latest position, within the context
-  const int32_t nblocks =
-      gmax < 0 ? 0 : min((gmax + kKeyBlock) / kKeyBlock, (int32_t(a.nk) + kKeyBlock - 1) / kKeyBlock);
+  // blocks up to the latest position, within the context: this workgroup's
+  // range of them, and keys, positions and the context's end from its first
+  // key on (a row that sees no key of the range's first block sees none of
+  // the range)
+  const uint32_t tile_blocks =
+      gmax < 0 ? 0u : uint32_t(min((gmax + kKeyBlock) / kKeyBlock, (int32_t(a.nk) + kKeyBlock - 1) / kKeyBlock));
+  const int32_t b_lo = __builtin_amdgcn_readfirstlane(int32_t(uint64_t(tile_blocks) * split / S));
+  const int32_t nblocks = __builtin_amdgcn_readfirstlane(int32_t(uint64_t(tile_blocks) * (split + 1) / S)) - b_lo;
+  const int32_t key0 = b_lo * kKeyBlock;
+  const int32_t nk = int32_t(a.nk) - key0;
+  const uint16_t* const k_range = a.k + int64_t(key0) * a.k_stride;
+  const uint16_t* const v_range = a.v + int64_t(key0) * a.v_stride;
+#pragma unroll
+  for (int t = 0; t < RT; ++t) rpos[t] -= key0;
+  wmax -= key0;
+  wmin -= key0;
 
   // per row tile: the reference max m (log2 units), -m for the exponents
   // (0 while m is -inf), and the logit above which m is raised,
@@ -363,7 +383,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     koff[j] = uint32_t((krow[j] * a.k_stride + kvh * D + piece * 8) * 2);
     voff[j] = uint32_t((krow[j] * a.v_stride + kvh * D + piece * 8) * 2);
   }
-  // K of block b into K buffer b % 3, V of block b into V buffer b % 3
+  // K of block b into K buffer b % kBuffers, V of block b into V buffer b % kBuffers
   // (clamped: a request past the end repeats the last block); rows past nk
   // of the last block repeat its last key (masked)
   auto request = [&](int32_t b, const uint16_t* src, int64_t stride, const uint32_t (&offs)[kInsts],
@@ -372,11 +392,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     b = min(b, nblocks - 1);
     const int32_t k0 = b * kKeyBlock;
     const uint16_t* base = src + int64_t(k0) * stride;
-    if (k0 + kKeyBlock <= int32_t(a.nk)) {
+    if (k0 + kKeyBlock <= nk) {
 #pragma unroll
       for (uint32_t j = 0; j < kInsts; ++j) lds_dma16(base, offs[j], l + (wave * kInsts + j) * 1024);
     } else {
-      const uint32_t last = uint32_t(int32_t(a.nk) - 1 - k0);
+      const uint32_t last = uint32_t(nk - 1 - k0);
 #pragma unroll
       for (uint32_t j = 0; j < kInsts; ++j) {
         const uint32_t back = krow[j] - min(krow[j], last);  // rows to step back past nk
@@ -390,7 +410,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   // takes its part in the requests and barriers).
   const int32_t wmin_s = __builtin_amdgcn_readfirstlane(wmin), wmax_s = __builtin_amdgcn_readfirstlane(wmax);
   const int32_t b_w = wmax_s < 0 ? 0 : min(wmax_s / kKeyBlock + 1, nblocks);
-  const int32_t b_m = wmax_s < 0 ? 0 : min(int32_t((int64_t(wmin_s) + 1) / kKeyBlock), b_w);
+  const int32_t b_m = wmax_s < 0 ? 0 : min(int32_t((int64_t(max(wmin_s, -1)) + 1) / kKeyBlock), b_w);
   // Software pipeline: step b takes S^T of block b + 1 on the MFMAs while
   // the VALU turns block b's S^T into logits, then P . V of block b - 1
   // while the VALU turns block b's logits into probabilities: the matrix
@@ -398,7 +418,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   // (MFMA/VALU co-execution 23% -> 42% of the MFMA busy time; under the
   // power limit the clock fell 6%, so 2.11-2.12 -> 2.05-2.07 ms per C3 layer
   // in same-box runs). K(b + 1) and V(b - 1) are read in step b. The loops
-  // take six steps at a time, so that the ring buffers and the register sets
+  // take four steps at a time, so that the ring buffers and the register sets
   // of every step are known at compile time: no per-read address adds
   // (1.99 -> 1.93 ms per C3 layer in same-box runs).
   // Lazy rescaling: exponents stay relative to a reference max m that is
@@ -425,15 +445,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
       ol[t][0] *= ao[0]; ol[t][1] *= ao[1]; ol[t][2] *= ao[2]; ol[t][3] *= ao[3];
     }
   };
-  // The steps' request streams: K three blocks ahead of the step, V one,
-  // clamped at the last block (every block before it is whole). Block j's K
-  // goes to K buffer j % 3, its V to V buffer j % 3 (kVOffset bytes after
-  // that K buffer).
+  // The steps' request streams: K kBuffers blocks ahead of the step, V two
+  // fewer, clamped at the last block (every block before it is whole). Block
+  // j's K goes to K buffer j % kBuffers, its V to V buffer j % kBuffers
+  // (kVOffset bytes after that K buffer).
   constexpr uint32_t kSlot = kKeyBlock * D * 2, kVOffset = kBuffers * kSlot;
   const int64_t kstep = int64_t(kKeyBlock) * a.k_stride * 2, vstep = int64_t(kKeyBlock) * a.v_stride * 2;
-  const bool last_whole = nblocks * kKeyBlock <= int32_t(a.nk);
-  const char* const kg0 = reinterpret_cast<const char*>(a.k) + int64_t(min(3, nblocks - 1)) * kstep;
-  const char* const vg0 = reinterpret_cast<const char*>(a.v) + int64_t(min(1, nblocks - 1)) * vstep;
+  const bool last_whole = nblocks * kKeyBlock <= nk;
+  const char* const kg0 = reinterpret_cast<const char*>(k_range) + int64_t(min(kBuffers, nblocks - 1)) * kstep;
+  const char* const vg0 = reinterpret_cast<const char*>(v_range) + int64_t(min(kBuffers - 2, nblocks - 1)) * vstep;
   const char* kg = kg0;
   const char* vg = vg0;
   auto stream = [&](int32_t j, const char*& g, int64_t stride_bytes, int64_t stride, const uint32_t (&offs)[kInsts],
@@ -443,7 +463,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
 #pragma unroll
       for (uint32_t i = 0; i < kInsts; ++i) lds_dma16(g, offs[i], l + (wave * kInsts + i) * 1024);
     } else {
-      const uint32_t last = uint32_t(int32_t(a.nk) - 1 - (nblocks - 1) * kKeyBlock);
+      const uint32_t last = uint32_t(nk - 1 - (nblocks - 1) * kKeyBlock);
 #pragma unroll
       for (uint32_t i = 0; i < kInsts; ++i) {
         const uint32_t back = krow[i] - min(krow[i], last);  // rows to step back past nk
@@ -453,7 +473,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     if (inner) g += stride_bytes;
   };
   // KIND: 0 visible, 1 masked, 2 P . V of the wave's last block only, 3 no
-  // work; FIRST: no block before; PHASE: b % 6 when known at compile time
+  // work; FIRST: no block before; PHASE: b % kPhases when known at compile time
   // (then every LDS address is a lane's offset plus a constant the DS
   // instruction's offset field carries), or -1. sc holds S^T of block b, pp
   // P of block b - 1; the step leaves S^T of block b + 1 in sn and P of
@@ -466,25 +486,25 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     constexpr bool FIRST = decltype(first)::value;
     constexpr int PHASE = decltype(phase)::value;
     constexpr bool FIX = decltype(fix)::value;
-    CBK_WAIT_VM_LGKM0(2 * kInsts);  // K(b + 1) and V(b - 1) have landed
+    // K(b + 1) and V(b - 1) have landed: all but the requests of the last kBuffers - 2 steps
+    CBK_WAIT_VM_LGKM0(2 * (kBuffers - 2) * kInsts);
     asm volatile("s_barrier" ::: "memory");
     uint32_t kb_addr, vb_addr, kw_addr, vw_addr;
     if constexpr (PHASE >= 0) {
-      kw_addr = lds_address(kbuf[PHASE % 3]);
-      vw_addr = lds_address(vbuf[(PHASE + 1) % 3]);
-      kb_addr = lds_address(kbuf[(PHASE + 1) % 3]);
-      vb_addr = lds_address(vbuf[(PHASE + 2) % 3]);
+      kw_addr = lds_address(kbuf[PHASE % kBuffers]);
+      vw_addr = lds_address(vbuf[(PHASE + kBuffers - 2) % kBuffers]);
+      kb_addr = lds_address(kbuf[(PHASE + 1) % kBuffers]);
+      vb_addr = lds_address(vbuf[(PHASE + kBuffers - 1) % kBuffers]);
     } else {
-      const uint32_t r = uint32_t(b) % 3;
       const uint32_t k0 = lds_address(kbuf[0]);
-      kw_addr = k0 + r * kSlot;
-      kb_addr = k0 + (r == 2 ? 0 : r + 1) * kSlot;
-      vw_addr = kb_addr + kVOffset;
-      vb_addr = k0 + (r == 0 ? 2 : r - 1) * kSlot + kVOffset;
+      kw_addr = k0 + (uint32_t(b) % kBuffers) * kSlot;
+      kb_addr = k0 + (uint32_t(b + 1) % kBuffers) * kSlot;
+      vw_addr = k0 + (uint32_t(b + kBuffers - 2) % kBuffers) * kSlot + kVOffset;
+      vb_addr = k0 + (uint32_t(b + kBuffers - 1) % kBuffers) * kSlot + kVOffset;
       asm volatile("" : "+s"(kb_addr), "+s"(vb_addr));
     }
-    stream(b + 3, kg, kstep, a.k_stride, koff, kw_addr);  // into the K buffer block b used
-    stream(b + 1, vg, vstep, a.v_stride, voff, vw_addr);  // into the V buffer block b - 2 used
+    stream(b + kBuffers, kg, kstep, a.k_stride, koff, kw_addr);  // into the K buffer block b used
+    stream(b + kBuffers - 2, vg, vstep, a.v_stride, voff, vw_addr);  // into the V buffer block b - 2 used
     if constexpr (KIND < 3) {
       const uint16_t* ks = (const uint16_t*)(__attribute__((address_space(3))) const uint16_t*)(size_t)kb_addr;
       const uint16_t* vs = (const uint16_t*)(__attribute__((address_space(3))) const uint16_t*)(size_t)vb_addr;
@@ -516,7 +536,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
               const float mn = fmaxf(m[t], bm * kLog2e + 1.f);  // +1: covers the second rounding
               alpha[t] = mn == kNegInf ? 1.f : __builtin_amdgcn_exp2f(m[t] - mn);
               m[t] = mn;
-              nms[t] = -mn;
+              nms[t] = mn == kNegInf ? 0.f : -mn;  // a row that sees no key of the range yet
               thr[t] = (mn + kRescale) * kLn2;
               pending = true;
             }
@@ -557,18 +577,21 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
       pa[t] = pb[t];
     }
   };
-  // steps [b, end) of one kind: six at a time from a multiple of 6 (the
-  // three-buffer rings and the two register sets back where they started),
-  // single steps at the edges
+  // steps [b, end) of one kind: kPhases at a time from a multiple of kPhases
+  // (the rings and the two register sets back where they started), single
+  // steps at the edges; the rare second pass takes single steps only (each
+  // copy of a step is 2.5 KB of code)
+  constexpr int kPhases = 4;
+  static_assert(kPhases % kBuffers == 0 && kPhases % 2 == 0, "whole turns of the rings and register sets");
   auto run = [&](auto kind, auto fix, int32_t& b, int32_t end) __attribute__((always_inline)) {
-    while (b < end && b % 6 != 0) single(kind, fix, b);
-    for (; b + 6 <= end; b += 6) {
-      step(kind, no(), std::integral_constant<int, 0>(), fix, b, sa, sb, pa, pb);
-      step(kind, no(), std::integral_constant<int, 1>(), fix, b + 1, sb, sa, pb, pa);
-      step(kind, no(), std::integral_constant<int, 2>(), fix, b + 2, sa, sb, pa, pb);
-      step(kind, no(), std::integral_constant<int, 3>(), fix, b + 3, sb, sa, pb, pa);
-      step(kind, no(), std::integral_constant<int, 4>(), fix, b + 4, sa, sb, pa, pb);
-      step(kind, no(), std::integral_constant<int, 5>(), fix, b + 5, sb, sa, pb, pa);
+    if constexpr (decltype(fix)::value) {
+      while (b < end && b % kPhases != 0) single(kind, fix, b);
+      for (; b + kPhases <= end; b += kPhases) {
+        step(kind, no(), std::integral_constant<int, 0>(), fix, b, sa, sb, pa, pb);
+        step(kind, no(), std::integral_constant<int, 1>(), fix, b + 1, sb, sa, pb, pa);
+        step(kind, no(), std::integral_constant<int, 2>(), fix, b + 2, sa, sb, pa, pb);
+        step(kind, no(), std::integral_constant<int, 3>(), fix, b + 3, sb, sa, pb, pa);
+      }
     }
     while (b < end) single(kind, fix, b);
   };
@@ -576,13 +599,17 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   // sets each row's reference from block 0, where every row with a position
   // sees key 0 at least)
   auto pass = [&](auto fix) __attribute__((always_inline)) {
-    // K of blocks 0-2 and V of block 0 ahead of step 0; then every wave
-    // takes steps 0 .. nblocks (the requests and barriers of each)
-    request(0, a.k, a.k_stride, koff, kbuf);
-    request(1, a.k, a.k_stride, koff, kbuf);
-    request(2, a.k, a.k_stride, koff, kbuf);
-    request(0, a.v, a.v_stride, voff, vbuf);
-    CBK_WAIT_VM_LGKM0(3 * kInsts);  // K(0) has landed
+    // the first kBuffers blocks of K and two fewer of V ahead of step 0, in
+    // the order the steps wait for them; then every wave takes steps 0 ..
+    // nblocks (the requests and barriers of each)
+    request(0, k_range, a.k_stride, koff, kbuf);
+    request(1, k_range, a.k_stride, koff, kbuf);
+#pragma unroll
+    for (int j = 0; j < kBuffers - 2; ++j) {
+      request(2 + j, k_range, a.k_stride, koff, kbuf);
+      request(j, v_range, a.v_stride, voff, vbuf);
+    }
+    CBK_WAIT_VM_LGKM0((2 * (kBuffers - 2) + 1) * kInsts);  // K(0) has landed
     asm volatile("s_barrier" ::: "memory");
     if (b_w > 0) {
       qk_block<F16, D, RT>((const uint16_t*)(__attribute__((address_space(3))) const uint16_t*)(size_t)lds_address(
@@ -590,19 +617,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
                            off, qf, sa);
     }
     int32_t b = 0;
-    auto first = [&](auto kind) __attribute__((always_inline)) {
-      step(kind, yes(), any(), no(), b++, sa, sb, pa, pb);
+    if (b_w > 0) {  // the masked form, whatever the block: one copy of the step fewer
+      step(masked(), yes(), any(), no(), b++, sa, sb, pa, pb);
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
         sa[t][0] = sb[t][0];
         sa[t][1] = sb[t][1];
         pa[t] = pb[t];
       }
-    };
-    if (b_m > 0)
-      first(visible());
-    else if (b_w > 0)
-      first(masked());
+    }
     run(visible(), fix, b, b_m);
     run(masked(), fix, b, b_w);
     if (b_w > 0)
@@ -654,6 +677,24 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   }
   __syncthreads();  // every wave is done with the K buffers the output staging reuses
 
+  if (S > 1) {  // this range's partial results (attention_split.hpp)
+    const uint64_t rows_all = uint64_t(a.nq) * a.hq;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float rm = __shfl(m[t], int(4 * grp + i));
+        const uint32_t rr = r_wave + 16 * t + 4 * grp + i;
+        if (rr >= nrows) continue;
+        const uint64_t id = split * rows_all + uint64_t(rr / a.group) * a.hq + kvh * a.group + rr % a.group;
+        if (row == 0) a.parts.ml[id] = make_float2(rm, ol[t][i]);
+        float* po = a.parts.o + id * D + row;
+        if (nblocks > 0)
+#pragma unroll
+          for (int c = 0; c < D / 16; ++c) po[16 * c] = o[t][c][i];
+      }
+    return;
+  }
   // normalize and write, one row tile at a time through the wave's LDS
   // staging area (the K buffers are free now): whole 16-byte pieces per row
   uint16_t* os = &kvbuf[0][0][0] + wave * 16 * D;
@@ -696,11 +737,11 @@ namespace cbk {
 namespace {
 
 // Key ranges of a launch (attn_splits) for inputs that passed the checks.
-uint32_t launch_splits(int64_t nq, int64_t nk, int64_t hq, int64_t hkv, int32_t dtype) {
-  if (dtype != CBK_DTYPE_F32) return 1;
+uint32_t launch_splits(int64_t nq, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim, int32_t dtype) {
   const uint64_t nrows = uint64_t(nq) * uint64_t(hq / hkv);
-  const uint64_t groups = (nrows + kAttnF32Rows - 1) / kAttnF32Rows * uint64_t(hkv);
-  return attn_splits(groups, kAttnF32PerCu, nk);
+  const uint64_t rows_per_wg = dtype == CBK_DTYPE_F32 ? kAttnF32Rows : 16 * kRowTiles * kWaves;
+  const uint64_t groups = (nrows + rows_per_wg - 1) / rows_per_wg * uint64_t(hkv);
+  return attn_splits(groups, dtype == CBK_DTYPE_F32 ? kAttnF32PerCu : per_cu(head_dim), nk);
 }
 
 int check_sizes(int64_t nq, int64_t nk, int64_t hq, int64_t hkv) {
@@ -771,11 +812,12 @@ int blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int64_t
   a.group = uint32_t(hq / hkv);
   a.d = uint32_t(head_dim);
   a.scale = scale;
+  a.parts = parts;
   const uint64_t nrows = uint64_t(nq) * uint64_t(a.group);
   constexpr int RT = kRowTiles;
   const uint32_t waves = kWaves;
   const uint64_t rows_per_wg = 16 * RT * uint64_t(waves);
-  const uint64_t groups = (nrows + rows_per_wg - 1) / rows_per_wg * uint64_t(hkv);
+  const uint64_t groups = (nrows + rows_per_wg - 1) / rows_per_wg * uint64_t(hkv) * parts.splits;
   CBK_REQUIRE(groups * 64 * waves < (uint64_t(1) << 32), "blend attention: %llu workgroups exceed one launch",
               (unsigned long long)groups);
   const dim3 grid(static_cast<uint32_t>(groups)), block(64 * waves);
@@ -787,7 +829,9 @@ int blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int64_t
     if (f16) hipLaunchKernelGGL((attn_kernel<true, 64, RT>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((attn_kernel<false, 64, RT>), grid, block, 0, s, a);
   }
-  return launch_status("blend attention");
+  if (int rc = launch_status("blend attention")) return rc;
+  if (parts.splits == 1) return CBK_OK;
+  return launch_attn_merge(parts, a.nq, a.hq, a.d, q_pos_dev, out_dev, out_row_stride_elems, dtype, false, s);
 }
 
 }  // namespace
@@ -799,7 +843,7 @@ size_t cbk_blend_attention_workspace_bytes(int64_t nq, int64_t nk, int64_t hq, i
                                            int32_t dtype) {
   using namespace cbk;
   if (check_sizes(nq, nk, hq, hkv) || nq == 0 || head_dim <= 0 || head_dim > 128) return 0;
-  return attn_parts_bytes(launch_splits(nq, nk, hq, hkv, dtype), uint64_t(nq) * uint64_t(hq), head_dim);
+  return attn_parts_bytes(launch_splits(nq, nk, hq, hkv, head_dim, dtype), uint64_t(nq) * uint64_t(hq), head_dim);
 }
 
 int cbk_blend_attention_ws(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev, int64_t nq,
@@ -815,7 +859,7 @@ int cbk_blend_attention_ws(const void* q_dev, int64_t q_row_stride_elems, const 
   uint32_t splits = 1;
   const uint64_t rows = uint64_t(nq) * uint64_t(hq);
   if (workspace_dev != nullptr) {
-    splits = launch_splits(nq, nk, hq, hkv, dtype);
+    splits = launch_splits(nq, nk, hq, hkv, head_dim, dtype);
     if (workspace_bytes < attn_parts_bytes(splits, rows, head_dim))
       return set_error(CBK_ERR_WORKSPACE, "attention workspace %zu < %zu bytes", workspace_bytes,
                        attn_parts_bytes(splits, rows, head_dim));

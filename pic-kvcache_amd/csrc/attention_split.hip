@@ -15,86 +15,84 @@ constexpr uint32_t kMaxSplits = 32;
 constexpr int64_t kMinKeysPerSplit = 128;
 constexpr int kMergeThreads = 256;
 
-__device__ __forceinline__ void store4(float* p, const float (&v)[4]) {
-  *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
-__device__ __forceinline__ void store4(__hip_bfloat16* p, const float (&v)[4]) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-  *reinterpret_cast<b4*>(p) = __builtin_convertvector((f4){v[0], v[1], v[2], v[3]}, b4);
-}
-__device__ __forceinline__ void store4(__half* p, const float (&v)[4]) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  *reinterpret_cast<h4*>(p) = __builtin_convertvector((f4){v[0], v[1], v[2], v[3]}, h4);
-}
-__device__ __forceinline__ void store1(float* p, float v) { *p = v; }
-__device__ __forceinline__ void store1(__hip_bfloat16* p, float v) { *p = __float2bfloat16(v); }
-__device__ __forceinline__ void store1(__half* p, float v) { *p = __float2half(v); }
+template <typename T> __device__ __forceinline__ T to_out(float v);
+template <> __device__ __forceinline__ float to_out<float>(float v) { return v; }
+template <> __device__ __forceinline__ __hip_bfloat16 to_out<__hip_bfloat16>(float v) { return __float2bfloat16(v); }
+template <> __device__ __forceinline__ __half to_out<__half>(float v) { return __float2half(v); }
 
-// One thread per (row, 4 dims): V of them per load where d and the output
-// allow it (VEC), element by element otherwise. The partials were written by
-// the launch before and are mostly still in the L2s and the last-level cache.
-template <typename T, bool VEC>
+// 32 lanes per row. Lane s weighs range s, so a row's maximum and sum are
+// lane reductions; then every lane sums N dims over the ranges with all the
+// ranges' loads independent (one thread that read a row's ranges one after
+// another took 0.3 us a range). N dims per lane: 4 at d = 128, 2 at 64, both
+// one load; 0: any d, dims 32 apart.
+template <typename T, int N>
 __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(const AttnParts parts, uint32_t nq, uint32_t hq,
                                                                    uint32_t d, const int64_t* pos, T* out,
                                                                    int64_t out_stride, bool nan_empty) {
-  const uint32_t per_row = (d + 3) / 4;
-  const uint64_t i = uint64_t(blockIdx.x) * kMergeThreads + threadIdx.x;
+  constexpr int E = N ? N : 4;  // d <= 128
+  typedef float VecN __attribute__((ext_vector_type(E)));
+  const uint32_t lane = threadIdx.x & 31;
   const uint64_t rows = uint64_t(nq) * hq;
-  const uint64_t row = i / per_row;
-  if (row >= rows) return;
-  const uint32_t dim = uint32_t(i - row * per_row) * 4;
-  float m = -__builtin_inff();
-  for (uint32_t s = 0; s < parts.splits; ++s) m = fmaxf(m, parts.ml[s * rows + row].x);
-  const float ms = m == -__builtin_inff() ? 0.f : m;
-  float l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (uint32_t s = 0; s < parts.splits; ++s) {
-    const float2 ml = parts.ml[s * rows + row];
-    const float* o = parts.o + (s * rows + row) * d + dim;
-    if (ml.y == 0.f) continue;  // no visible keys: its output was not written
-    const float w = __builtin_amdgcn_exp2f(ml.x - ms);
-    l += w * ml.y;
-    if constexpr (VEC) {
-      const float4 v = *reinterpret_cast<const float4*>(o);
-      acc[0] = fmaf(w, v.x, acc[0]);
-      acc[1] = fmaf(w, v.y, acc[1]);
-      acc[2] = fmaf(w, v.z, acc[2]);
-      acc[3] = fmaf(w, v.w, acc[3]);
+  const uint64_t row = uint64_t(blockIdx.x) * (kMergeThreads / 32) + (threadIdx.x >> 5);
+  if (row >= rows) return;  // both halves' exchanges stay within their 32 lanes
+  const uint32_t S = parts.splits;
+  const float2 ml = lane < S ? parts.ml[lane * rows + row] : make_float2(-__builtin_inff(), 0.f);
+  float m = ml.x;
+#pragma unroll
+  for (int off = 16; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 32));
+  // a range without visible keys for the row: its sum is 0, its output may be unwritten
+  const float w = ml.y == 0.f ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+  float l = ml.y == 0.f ? 0.f : w * ml.y;
+#pragma unroll
+  for (int off = 16; off >= 1; off >>= 1) l += __shfl_xor(l, off, 32);
+  float acc[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) acc[e] = 0.f;
+  const float* o = parts.o + row * d;
+#pragma unroll 8
+  for (uint32_t s = 0; s < S; ++s) {
+    const float ws = __shfl(w, int(s), 32);
+    const bool used = ws != 0.f;
+    if constexpr (N != 0) {
+      const VecN v = used ? *reinterpret_cast<const VecN*>(o + s * rows * d + lane * N) : VecN(0.f);
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[e] = fmaf(ws, v[e], acc[e]);
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (dim + e < d) acc[e] = fmaf(w, o[e], acc[e]);
+      for (int e = 0; e < E; ++e)
+        if (used && lane + 32 * e < d) acc[e] = fmaf(ws, o[s * rows * d + lane + 32 * e], acc[e]);
     }
   }
   const uint32_t q = uint32_t(row / hq), h = uint32_t(row - uint64_t(q) * hq);
   const float empty = nan_empty && pos[q] >= 0 ? __uint_as_float(0x7fc00000u) : 0.f;
   const float inv = 1.f / l;
-  T* dst = out + int64_t(q) * out_stride + int64_t(h) * d + dim;
+  T* dst = out + int64_t(q) * out_stride + int64_t(h) * d;
+  T res[E];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) acc[e] = l == 0.f ? empty : acc[e] * inv;
-  if constexpr (VEC) {
-    store4(dst, acc);
+  for (int e = 0; e < E; ++e) res[e] = to_out<T>(l == 0.f ? empty : acc[e] * inv);
+  if constexpr (N != 0) {
+    using V = typename Vec<int(N * sizeof(T))>::T;
+    *reinterpret_cast<V*>(dst + lane * N) = *reinterpret_cast<const V*>(res);
   } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (dim + e < d) store1(dst + e, acc[e]);
+    for (int e = 0; e < E; ++e)
+      if (lane + 32 * e < d) dst[lane + 32 * e] = res[e];
   }
 }
 
 template <typename T>
 int launch_merge_t(const AttnParts& parts, uint32_t nq, uint32_t hq, uint32_t d, const int64_t* pos, T* out,
                    int64_t out_stride, bool nan_empty, hipStream_t stream) {
-  const uint64_t threads = uint64_t(nq) * hq * ((d + 3) / 4);
-  const dim3 grid(uint32_t((threads + kMergeThreads - 1) / kMergeThreads));
-  const bool vec = d % 4 == 0 && out_stride % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(T)) == 0;
-  if (vec)
-    hipLaunchKernelGGL((attn_merge_kernel<T, true>), grid, dim3(kMergeThreads), 0, stream, parts, nq, hq, d, pos,
-                       out, out_stride, nan_empty);
-  else
-    hipLaunchKernelGGL((attn_merge_kernel<T, false>), grid, dim3(kMergeThreads), 0, stream, parts, nq, hq, d, pos,
-                       out, out_stride, nan_empty);
+  constexpr uint64_t kRows = kMergeThreads / 32;
+  const dim3 grid(uint32_t((uint64_t(nq) * hq + kRows - 1) / kRows));
+  const bool aligned = out_stride % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(T)) == 0;
+#define CBK_MERGE(N)                                                                                             \
+  hipLaunchKernelGGL((attn_merge_kernel<T, N>), grid, dim3(kMergeThreads), 0, stream, parts, nq, hq, d, pos, out, \
+                     out_stride, nan_empty)
+  if (d == 128 && aligned) CBK_MERGE(4);
+  else if (d == 64 && aligned) CBK_MERGE(2);
+  else CBK_MERGE(0);
+#undef CBK_MERGE
   return launch_status("attention merge");
 }
 
@@ -104,7 +102,10 @@ uint32_t attn_splits(uint64_t groups, uint32_t per_cu, int64_t nk) {
   int cus = 0;
   if (groups == 0 || device_cus(&cus)) return 1;
   const uint64_t want = uint64_t(per_cu) * uint32_t(cus);
-  uint64_t s = (want + groups - 1) / groups;
+  // one round of workgroups where that takes three or more ranges; with fewer
+  // the ranges are long, and two shorter rounds even out the tiles' lengths
+  uint64_t s = want / groups;
+  if (s < 3) s = 2 * want / groups;
   s = std::min<uint64_t>(s, uint64_t(nk / kMinKeysPerSplit));
   return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(s, kMaxSplits)));
 }

@@ -8,6 +8,8 @@
 
 namespace cbk {
 
+constexpr int kAttnKeyBlock = 32;  // keys per block of the attention kernels
+
 // Partial results of `splits` key ranges: for range s and row r = query *
 // hq + head, ml[s * rows + r] = (maximum in log2 units, sum of 2^(x - maximum))
 // and o[(s * rows + r) * d ..] the sum of 2^(x - maximum) * value, float32.
@@ -17,8 +19,18 @@ struct AttnParts {
   float* o;
 };
 
-// The ranges that bring a launch of `groups` workgroups to about `per_cu`
-// workgroups per CU (1 where it has as many without), and the partials' bytes.
+// The ranges of a launch of `groups` workgroups (1: none), so that about
+// `per_cu` workgroups per CU run at once, and the partials' bytes. us a call
+// at 1 / 2 / 3 / 4 / 6 / 8 / 10 / 16 ranges, D 128, in groups without ranges:
+//   48 (180 queries of 8191 keys, 32 heads over 8)  167 / 94 / 69 / 57 / 44 / 41 / 38 / 47
+//  104 (400 of 2000, 32 over 8)                      48 / 37 / 35 / 34 / 37 / 39 / 44 / 53
+//  128 (500 of 4095, 32 over 4)                      89 / 57 / 47 / 43 / 50 / 50 / 57 / 73
+//  248 (990 of 4095, 32 over 8, f16)                 94 / 74 / 73 / 72 / 80 / 89
+//  256 (1000 of 32767, 32 over 8)                   648 / 371 / 337 / 330 / 336 / 344 / 357 / 398
+//  376 (3000 of 16000, 16 over 8)                   333 / 243 / 239 / 242 / 260 / 283 / 307 / 388
+//  500 (2000 of 12000, 32 over 4, f16)              277 / 251 / 250 / 259 / 279 / 309
+// 1752 (7000 of 32767, 32 over 4)                  1860 / 1894 / - / 1972 / - / 2186
+// A range more costs its partials' traffic: 16 MB each way a range and 32K rows.
 uint32_t attn_splits(uint64_t groups, uint32_t per_cu, int64_t nk);
 size_t attn_parts_bytes(uint32_t splits, uint64_t rows, int64_t d);
 AttnParts attn_parts(uint32_t splits, uint64_t rows, void* workspace);

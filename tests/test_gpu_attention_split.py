@@ -98,3 +98,48 @@ def test_f32_values_past_a_position_do_not_reach_its_row():
     assert np.all(np.abs(got - want)[clean] <= _f32_bound(mass, size, d, nk, 0.125)[clean])
     assert np.all(got[pos.numpy() < 0] == 0)
     assert np.all(np.isnan(got[pos.numpy() >= 300]))
+
+
+# 16-bit rows around the 128-row tile, keys around the 32-key block and the
+# four-block rings, ranges in which rows see nothing, and both merge widths;
+# keys and queries in {-1, 0, 1} / 8, whose dot products are exact
+@pytest.mark.parametrize("nq,nk,hq,hkv,d,dtype", [
+    (1, 1, 1, 1, 128, torch.bfloat16), (1, 4097, 8, 8, 128, torch.bfloat16), (33, 1023, 4, 1, 64, torch.float16),
+    (31, 700, 8, 2, 128, torch.float16), (129, 255, 1, 1, 64, torch.bfloat16), (64, 8191, 2, 2, 64, torch.bfloat16),
+    (300, 3000, 16, 8, 128, torch.bfloat16), (17, 161, 5, 1, 128, torch.bfloat16),
+])
+def test_16_bit_matches_float64(nq, nk, hq, hkv, d, dtype):
+    g = torch.Generator().manual_seed(nq)
+    q, k = ((torch.randint(-1, 2, (n, h, d), generator=g) / 8).to(dtype) for n, h in ((nq, hq), (nk, hkv)))
+    v = torch.randn(nk, hkv, d, generator=g).to(dtype)
+    pos = torch.randint(0, nk, (nq,), generator=g)
+    pos[-1] = nk - 1
+    want, mass, _ = _f64(q, k, v, pos, 1.0)
+    got = blend_attention(q.to(DEV), k.to(DEV), v.to(DEV), pos.to(DEV), 1.0).float().cpu().numpy()
+    # the probabilities, their sum's terms and the output are each rounded once
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert np.all(np.abs(got - want) <= 3 * u * mass + 1e-6)
+
+
+def test_ranges_agree_with_one_range_far_above_the_first_blocks_maximum():
+    # logits that outgrow each range's first block (the online second pass),
+    # in some ranges only
+    nq, nk, hq, hkv, d = 40, 4000, 4, 1, 128
+    g = torch.Generator().manual_seed(3)
+    q = torch.ones(nq, hq, d).to(torch.bfloat16).to(DEV)
+    k = (torch.randint(-1, 2, (nk, hkv, d), generator=g) / 8).to(torch.bfloat16)
+    k[1500:1510] = 1.5
+    k[3900] = 2.0
+    v = torch.randn(nk, hkv, d, generator=g).to(torch.bfloat16).to(DEV)
+    pos = (torch.arange(nq) * 100 + 99).to(DEV)
+    k = k.to(DEV)
+    got = blend_attention(q, k, v, pos, 1.0)
+    out = torch.empty_like(got)
+    rc = _native.load().cbk_blend_attention(
+        q.data_ptr(), hq * d, pos.data_ptr(), nq, k.data_ptr(), hkv * d, v.data_ptr(), hkv * d, nk, hq, hkv, d,
+        1.0, _native.DTYPE_CODES[torch.bfloat16], out.data_ptr(), hq * d, _native.stream_handle(DEV))
+    _native.check(rc, "blend_attention")
+    diff = (got.float() - out.float()).abs()
+    assert torch.isfinite(got).all()
+    # each side rounds probabilities and outputs once: 2 * 2 * 2^-8 of values up to 4.5
+    assert float(diff.max()) <= 4 * 2.0 ** -8 * 4.5
