@@ -1,4 +1,4 @@
-// Sparse-Q attention-mass scores for gfx950 (the only MFMA kernel here).
+// Sparse-Q attention-mass scores for gfx950 .
 //
 // full[k] = sum_{h, q : pos_q >= k} softmax_k( r(Q[q,h] . K[k, h/G]) * scale )
 // where r rounds the dot product to the input dtype (the reference's bf16
@@ -31,14 +31,11 @@
 // 4*(i/8) + i%4. Q.K^T has both operands row-major in D, so A and B
 // fragments are the same 16-byte loads of 8 consecutive dims.
 //
-// A float32 path (no MFMA, exact float32 dots) serves float32 inputs.
-#include <hip/hip_bf16.h>
-#include <hip/hip_fp16.h>
-
+// float32 inputs: sparse_q_f32.hip.
 #include <algorithm>
 #include <type_traits>
 
-#include "cbk_common.hpp"
+#include "sparse_q.hpp"
 
 namespace cbk {
 namespace {
@@ -49,66 +46,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 256;
-constexpr int kQTile = 16;
 constexpr int kTileWords = 32;        // per query tile: 16 positions, min, max, unused
 constexpr int kKeyBlock1 = 64;        // keys per LDS block in rowstats
 constexpr int kColTiles = 4;          // 16-key column tiles per wave in colsum
 constexpr int kKeyBlock2 = 4 * 16 * kColTiles;  // 256 keys per colsum workgroup
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kNegInf = -__builtin_inff();
-
-struct SqArgs {
-  const char* q;          // [*, Hq, D] rows
-  int64_t q_stride;       // elements between query rows
-  const int64_t* q_index; // [nq] rows of q that are sparse queries (nullable: 0..nq-1)
-  const int64_t* pos;     // [*] absolute position of every q row (indexed like q)
-  const char* k;          // [nk, Hkv, D]
-  int64_t k_stride;       // elements between key rows
-  uint32_t nq, nk, hq, hkv, d, groups;
-  float c2;               // scale * log2(e)
-  int32_t round_mode;     // 0 none, 1 bf16, 2 f16
-  float2* stats;          // [hq][nq_pad] (m2 + log2(l), unused)
-  float2* chunk_stats;    // [row_chunks][hq][nq_pad] (m2, l) of each key range, row_chunks > 1
-  uint32_t row_chunks;    // key ranges per (query tile, kv head) in rowstats
-  int32_t* tiles;         // [nq_pad / 16][32]: the 16 query positions (-1 past nq), min, max, unused
-  float* partial;         // [hkv][nk]
-  uint16_t* qdense;       // [hkv][nq_pad / 16][groups][16][D]: query rows in colsum's unit order
-  uint32_t nq_pad;
-  uint32_t col_splits;    // query-unit ranges per (key block, kv head) in colsum
-};
-
-__device__ __forceinline__ float round_logit(float x, int mode) {
-  if (mode == 1) return __bfloat162float(__float2bfloat16(x));
-  if (mode == 2) return __half2float(__float2half(x));
-  return x;
-}
-
-__device__ __forceinline__ int32_t query_pos(const SqArgs& a, uint32_t qi) {
-  if (qi >= a.nq) return -1;
-  const int64_t row = a.q_index ? a.q_index[qi] : int64_t(qi);
-  return int32_t(a.pos[row]);
-}
-
-__device__ __forceinline__ const char* query_row(const SqArgs& a, uint32_t qi, uint32_t h, uint32_t es) {
-  const int64_t row = a.q_index ? a.q_index[qi] : int64_t(qi);
-  return a.q + (row * a.q_stride + int64_t(h) * a.d) * es;
-}
-
-// Published per (head, query) row: x = m + log2(l), so that a probability
-// is the single exp2(logit * scale * log2(e) - x) (+inf: an empty row).
-__device__ __forceinline__ float2 row_stats(float m, float l) {
-  return make_float2(l > 0.f ? m + log2f(l) : __builtin_inff(), 0.f);
-}
-
-// Online (max, sum) update in the log2 domain with -inf guards.
-__device__ __forceinline__ void stats_merge(float& m, float& l, float m_o, float l_o) {
-  const float mn = fmaxf(m, m_o);
-  const float ms = mn == kNegInf ? 0.f : mn;
-  l = l * __builtin_amdgcn_exp2f(m - ms) + l_o * __builtin_amdgcn_exp2f(m_o - ms);
-  m = mn;
-}
-
 template <typename V>
 __device__ __forceinline__ f32x4 mfma16(const V& a, const V& b, const f32x4& c);
 template <>
@@ -870,52 +811,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
   }
 }
 
-// ----------------------------------------------------------- float32 path
-
-// rowstats: one wavefront per (query, head); lanes stride over keys.
-__global__ __launch_bounds__(kThreads) void sq_rowstats_f32_kernel(const SqArgs a) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t item = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  if (item >= a.nq * a.hq) return;
-  const uint32_t qi = item / a.hq, h = item % a.hq, g = h / a.groups;
-  const int32_t pos = min(query_pos(a, qi), int32_t(a.nk) - 1);
-  const float* qrow = reinterpret_cast<const float*>(query_row(a, qi, h, 4));
-  float m = kNegInf, l = 0.f;
-  for (int32_t key = int32_t(lane); key <= pos; key += 64) {
-    const float* krow = reinterpret_cast<const float*>(a.k) + int64_t(key) * a.k_stride + int64_t(g) * a.d;
-    float dot = 0.f;
-    for (uint32_t e = 0; e < a.d; ++e) dot = fmaf(qrow[e], krow[e], dot);
-    const float x = round_logit(dot, a.round_mode) * a.c2;
-    stats_merge(m, l, x, 1.f);
-  }
-  for (int off = 1; off < 64; off <<= 1) {
-    const float mo = __shfl_xor(m, off, 64), lo = __shfl_xor(l, off, 64);
-    stats_merge(m, l, mo, lo);
-  }
-  if (lane == 0) a.stats[int64_t(h) * a.nq_pad + qi] = row_stats(m, l);
-}
-
-// colsum: one thread per (key, kv head), fixed query/head order.
-__global__ __launch_bounds__(kThreads) void sq_colsum_f32_kernel(const SqArgs a) {
-  const uint32_t t = blockIdx.x * kThreads + threadIdx.x;
-  if (t >= a.nk * a.hkv) return;
-  const uint32_t key = t % a.nk, g = t / a.nk;
-  const float* krow = reinterpret_cast<const float*>(a.k) + int64_t(key) * a.k_stride + int64_t(g) * a.d;
-  float acc = 0.f;
-  for (uint32_t qi = 0; qi < a.nq; ++qi) {
-    if (query_pos(a, qi) < int32_t(key)) continue;
-    for (uint32_t hl = 0; hl < a.groups; ++hl) {
-      const uint32_t h = g * a.groups + hl;
-      const float* qrow = reinterpret_cast<const float*>(query_row(a, qi, h, 4));
-      float dot = 0.f;
-      for (uint32_t e = 0; e < a.d; ++e) dot = fmaf(qrow[e], krow[e], dot);
-      const float2 st = a.stats[int64_t(h) * a.nq_pad + qi];
-      acc += __builtin_amdgcn_exp2f(round_logit(dot, a.round_mode) * a.c2 - st.x);
-    }
-  }
-  a.partial[int64_t(g) * a.nk + key] = acc;
-}
-
 // ---------------------------------------------------------------- gather
 
 // out / full = the sum over query-unit ranges and kv heads of the partial
@@ -948,11 +843,6 @@ __global__ void sq_zero_kernel(float* p, uint64_t n) {
 
 // Largest head_dim of the MFMA path: the dense query copy is sized for it.
 constexpr int64_t kMaxHeadDim = 128;
-
-// Key ranges a (query tile, kv head) of rowstats may be split into.
-constexpr uint32_t kMaxRowChunks = 8;
-// Query-unit ranges a (key block, kv head) of colsum may be split into.
-constexpr uint32_t kMaxColSplits = 4;
 
 struct SqLayout {
   uint32_t nq_pad, ntiles;
@@ -1052,8 +942,7 @@ int launch_mfma_ks(SqArgs& a, int cus, hipStream_t stream) {
   else
     hipLaunchKernelGGL((sq_rowstats_kernel<V, KS, 4, RMODE, false>), g1, dim3(kThreads), 0, stream, a);
   if (a.row_chunks > 1)
-    hipLaunchKernelGGL(sq_merge_kernel, dim3((a.hq * a.nq_pad + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                       stream, a);
+    launch_sq_merge(a, stream);
   // column-pass units: a tile's chunk of 4 heads when the group is a
   // multiple of 4, else four consecutive (tile, head) rows (spanning up to 4
   // tiles at one head per KV head, 2 otherwise); measured on 98,304-key
@@ -1088,6 +977,11 @@ int launch_mfma(SqArgs& a, int ksteps, hipStream_t stream) {
 }
 
 }  // namespace
+
+void launch_sq_merge(const SqArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL(sq_merge_kernel, dim3((a.hq * a.nq_pad + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, a);
+}
+
 }  // namespace cbk
 
 extern "C" {
@@ -1153,10 +1047,7 @@ int cbk_sparse_q_scores(const void* q_dev, int64_t q_row_stride_elems, const int
     hipLaunchKernelGGL(sq_zero_kernel, dim3(uint32_t(std::min<uint64_t>((n + kThreads - 1) / kThreads, 4096))),
                        dim3(kThreads), 0, s, a.partial, n);
   } else if (dtype == CBK_DTYPE_F32) {
-    const uint64_t items = uint64_t(nq) * hq;
-    hipLaunchKernelGGL(sq_rowstats_f32_kernel, dim3(uint32_t((items + 3) / 4)), dim3(kThreads), 0, s, a);
-    hipLaunchKernelGGL(sq_colsum_f32_kernel, dim3(uint32_t((uint64_t(nk) * hkv + kThreads - 1) / kThreads)),
-                       dim3(kThreads), 0, s, a);
+    if (int rc = launch_sq_f32(a, s)) return rc;
   } else {
     CBK_REQUIRE(dtype == CBK_DTYPE_BF16 || dtype == CBK_DTYPE_F16, "dtype %d", int(dtype));
     CBK_REQUIRE(head_dim % 32 == 0 && (head_dim == 64 || head_dim == 128),

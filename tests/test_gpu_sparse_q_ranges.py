@@ -1,0 +1,69 @@
+"""GPU parity of the Sparse-Q passes at the ends of their row tiles, key
+blocks and ranges, against float64."""
+
+import numpy as np
+import pytest
+import torch
+
+from cacheblend_vllm import selection as S
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def _f64(q, k, rows, pos, scale):
+    """(attention mass per key, largest sum_i |q_i k_i|) in float64."""
+    g = q.shape[1] // k.shape[1]
+    full, size = np.zeros(k.shape[0]), 0.0
+    visible = pos[rows].numpy()[:, None] >= np.arange(k.shape[0])[None, :]
+    for h in range(q.shape[1]):
+        qh, kh = q[rows, h].double().numpy(), k[:, h // g].double().numpy()
+        x = np.where(visible, qh @ kh.T * scale, -np.inf)
+        e = np.exp(x - x.max(axis=1, keepdims=True, initial=-1e300))
+        full += (e / np.maximum(e.sum(axis=1, keepdims=True), 1e-300)).sum(axis=0)
+        size = max(size, float((np.abs(qh) @ np.abs(kh).T).max()))
+    return full, size
+
+
+# query rows around the 64-row tile and the 32-row block, keys around the
+# 32-key block and 64-key tile, head sizes around the padded 64 and 128 (and
+# one above), rows in any order and at positions before the first key
+@pytest.mark.parametrize("nq,nk,hq,hkv,d", [
+    (1, 1, 1, 1, 64), (1, 65, 16, 1, 128), (31, 64, 2, 1, 64), (33, 63, 2, 2, 128), (65, 700, 3, 1, 100),
+    (22, 1031, 6, 2, 3), (64, 4097, 8, 4, 128), (130, 2047, 16, 8, 128), (40, 333, 10, 2, 66), (9, 200, 4, 2, 136),
+])
+def test_f32_matches_float64(nq, nk, hq, hkv, d):
+    g = torch.Generator().manual_seed(nq + nk)
+    n = 2 * nq
+    q, k = torch.randn(n, hq, d, generator=g), torch.randn(nk, hkv, d, generator=g)
+    pos = torch.randint(-1, nk, (n,), generator=g)
+    rows = torch.randperm(n, generator=g)[:nq]
+    pos[rows[0]] = nk - 1
+    scale = d ** -0.5
+    _, full = S.sparse_q_full_scores(q.to(DEV), k.to(DEV), rows.to(DEV), pos.to(DEV), scale, want_full=True)
+    want, size = _f64(q, k, rows, pos, scale)
+    # every term is positive; a logit is off by at most (d + 3) roundings of
+    # its absolute terms, twice in a probability (itself and its row's sum),
+    # and the row's sum, the exponentials and the score's sum by the rest
+    u = 2.0 ** -24
+    bound = np.expm1(2 * (d + 3) * u * size * scale) + (nk + nq * hq + 24 + 2 * size * scale) * u
+    err = np.abs(full.cpu().numpy() - want) / np.maximum(want, 1e-300)
+    print(f"largest error / bound {err.max() / bound:.3f}", flush=True)
+    assert err.max() <= bound
+
+
+def test_f32_unaligned_views():
+    # rows 4 bytes off a 16-byte boundary
+    nq, nk, hq, hkv, d = 50, 500, 4, 2, 64
+    g = torch.Generator().manual_seed(4)
+    q, k = torch.randn(nq, hq, d, generator=g), torch.randn(nk, hkv, d, generator=g)
+    pos = torch.arange(nk - nq, nk)
+
+    def off(t):
+        flat = torch.zeros(t.shape[0], t.shape[1] * d + 1)
+        flat[:, 1:] = t.reshape(t.shape[0], -1)
+        return flat.to(DEV)[:, 1:].unflatten(1, (t.shape[1], d))
+
+    _, want = S.sparse_q_full_scores(q.to(DEV), k.to(DEV), None, pos.to(DEV), 0.125, want_full=True)
+    _, got = S.sparse_q_full_scores(off(q), off(k), None, pos.to(DEV), 0.125, want_full=True)
+    assert torch.equal(got, want)
