@@ -135,6 +135,21 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
   return v;
 }
 
+// All-reduce of `v` over each group of 16 lanes by DPP (quad swaps, then the
+// mirrored half rows and rows): no LDS round trip, which four exchanges in
+// turn wait out.
+template <typename F>
+__device__ __forceinline__ float row16_reduce(float v, F op) {
+#define CBK_DPP_STEP(ctrl) \
+  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true)))
+  CBK_DPP_STEP(0xB1);   // quad_perm [1, 0, 3, 2]
+  CBK_DPP_STEP(0x4E);   // quad_perm [2, 3, 0, 1]
+  CBK_DPP_STEP(0x141);  // row_half_mirror
+  CBK_DPP_STEP(0x140);  // row_mirror
+#undef CBK_DPP_STEP
+  return v;
+}
+
 // Inclusive prefix sum over the 64 lanes of a wavefront.
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
   const int lane = threadIdx.x & 63;

@@ -285,25 +285,23 @@ void sq_rowstats_kernel(const SqArgs a) {
   const uint32_t q0 = qt * kQTile;
   if (threadIdx.x < kQTile * TPW) s_pos[threadIdx.x] = query_pos(a, qt_first * kQTile + threadIdx.x);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t lo = 0x7fffffff, hi = -1;
-    for (int u = 0; u < TPW; ++u) {
-      int32_t tlo = 0x7fffffff, thi = -1;
-      for (int i = 0; i < kQTile; ++i) {
-        if ((qt_first + u) * kQTile + i < a.nq) {
-          tlo = min(tlo, s_pos[u * kQTile + i]);
-          thi = max(thi, s_pos[u * kQTile + i]);
-        }
+  if (threadIdx.x < 64) {  // 16 lanes per tile; lanes past the workgroup's tiles repeat its first
+    const uint32_t u = lane / kQTile % TPW, i = lane % kQTile;
+    const bool have = (qt_first + u) * kQTile + i < a.nq;
+    int32_t lo = have ? s_pos[u * kQTile + i] : 0x7fffffff, hi = have ? s_pos[u * kQTile + i] : -1;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      if (off == kQTile && lane < kQTile * TPW && i == 0 && g == 0 && chunk == 0 && qt_first + u < ntiles_pad) {
+        a.tiles[kTileWords * (qt_first + u) + kQTile] = lo;
+        a.tiles[kTileWords * (qt_first + u) + kQTile + 1] = hi;
       }
-      lo = min(lo, tlo);
-      hi = max(hi, thi);
-      if (g == 0 && chunk == 0 && qt_first + u < ntiles_pad) {
-        a.tiles[kTileWords * (qt_first + u) + kQTile] = tlo;
-        a.tiles[kTileWords * (qt_first + u) + kQTile + 1] = thi;
-      }
+      lo = min(lo, __shfl_xor(lo, off, 64));
+      hi = max(hi, __shfl_xor(hi, off, 64));
     }
-    s_minmax[0] = lo;
-    s_minmax[1] = hi;
+    if (lane == 0) {
+      s_minmax[0] = lo;
+      s_minmax[1] = hi;
+    }
   }
   __syncthreads();
   // workgroup-uniform, and scalar: the key-block loop and its branches stay
@@ -465,11 +463,15 @@ void sq_rowstats_kernel(const SqArgs a) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
       float mm = m[t][i], ll = l[t][i];
-#pragma unroll
-      for (int off = WIDE ? 32 : 1; off < (WIDE ? 64 : 16); off <<= 1) {
-        const float mo = __shfl_xor(mm, off, 64);
-        const float lo = __shfl_xor(ll, off, 64);
+      if constexpr (WIDE) {
+        const float mo = __shfl_xor(mm, 32, 64);
+        const float lo = __shfl_xor(ll, 32, 64);
         stats_merge(mm, ll, mo, lo);
+      } else {
+        // the row's maximum over its 16 lanes, then their sums against it
+        mm = row16_reduce(mm, [](float x, float y) { return fmaxf(x, y); });
+        ll *= __builtin_amdgcn_exp2f(m[t][i] - (mm == kNegInf ? 0.f : mm));
+        ll = row16_reduce(ll, [](float x, float y) { return x + y; });
       }
       const int slot = WIDE ? 2 * t + int(rgrp & 1) : t;
       const uint32_t h = g * a.groups + wv + WT * slot;
@@ -484,17 +486,32 @@ void sq_rowstats_kernel(const SqArgs a) {
   }
 }
 
-// Merges the key ranges' (m2, l) of every (head, query) row in range order
-// (the same result run to run) and publishes m2 + log2(l).
+// Merges the key ranges' (m2, l) of every (head, query) row in a fixed order
+// (the same result run to run) and publishes m2 + log2(l): 64 rows per
+// workgroup, each wave a quarter of the ranges with 8 loads in flight (one
+// thread that took a row's ranges in turn: 4.7 us for 8 ranges).
 __global__ __launch_bounds__(kThreads) void sq_merge_kernel(const SqArgs a) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  __shared__ float2 part[kThreads / 64][64];
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t rows = a.hq * a.nq_pad;
-  if (i >= rows) return;
+  const uint32_t i = blockIdx.x * 64 + lane;
+  const uint32_t c_lo = a.row_chunks * wave / 4, c_hi = a.row_chunks * (wave + 1) / 4;
   float m = kNegInf, l = 0.f;
-  for (uint32_t c = 0; c < a.row_chunks; ++c) {
-    const float2 p = a.chunk_stats[int64_t(c) * rows + i];
-    stats_merge(m, l, p.x, p.y);
+  if (i < rows) {
+    for (uint32_t c = c_lo; c < c_hi; c += 8) {
+      float2 p[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u)
+        p[u] = c + u < c_hi ? a.chunk_stats[int64_t(c + u) * rows + i] : make_float2(kNegInf, 0.f);
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u) stats_merge(m, l, p[u].x, p[u].y);
+    }
   }
+  part[wave][lane] = make_float2(m, l);
+  __syncthreads();
+  if (wave != 0 || i >= rows) return;
+#pragma unroll
+  for (uint32_t w = 1; w < 4; ++w) stats_merge(m, l, part[w][lane].x, part[w][lane].y);
   a.stats[i] = row_stats(m, l);
 }
 
@@ -813,6 +830,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
 
 // ---------------------------------------------------------------- gather
 
+// The sum over `parts` partial column sums of key k, in that order, with 8
+// loads in flight.
+__device__ __forceinline__ float column_sum(const float* partial, uint32_t nk, uint32_t parts, uint32_t k) {
+  float v = 0.f;
+  for (uint32_t p = 0; p < parts; p += 8) {
+    float w[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) w[u] = p + u < parts ? partial[int64_t(p + u) * nk + k] : 0.f;
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) v += w[u];
+  }
+  return v;
+}
+
 // out / full = the sum over query-unit ranges and kv heads of the partial
 // column sums [splits][hkv][nk], in that order.
 __global__ __launch_bounds__(kThreads) void sq_gather_kernel(const float* partial, uint32_t nk, uint32_t hkv,
@@ -820,19 +851,11 @@ __global__ __launch_bounds__(kThreads) void sq_gather_kernel(const float* partia
                                                              float* out, float* full) {
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   const uint32_t parts = splits * hkv;
-  if (full != nullptr && i < nk) {
-    float v = 0.f;
-    for (uint32_t p = 0; p < parts; ++p) v += partial[int64_t(p) * nk + i];
-    full[i] = v;
-  }
+  if (full != nullptr && i < nk) full[i] = column_sum(partial, nk, parts, i);
   if (out != nullptr && i < n) {
     const int64_t k = index ? index[i] : int64_t(i);
-    float v = __uint_as_float(0x7fc00000u);
-    if (k >= 0 && k < int64_t(nk)) {
-      v = 0.f;
-      for (uint32_t p = 0; p < parts; ++p) v += partial[int64_t(p) * nk + k];
-    }
-    out[i] = v;
+    const bool ok = k >= 0 && k < int64_t(nk);
+    out[i] = ok ? column_sum(partial, nk, parts, uint32_t(k)) : __uint_as_float(0x7fc00000u);
   }
 }
 
@@ -864,7 +887,7 @@ __host__ SqLayout sq_layout(int64_t nq, int64_t nk, int64_t hq, int64_t hkv) {
   L.qdense = (L.partial + uint64_t(kMaxColSplits) * hkv * nk * 4 + 255) & ~uint64_t(255);
   // padded by one unit: a partial head chunk's requests read past its group
   L.chunk_stats = (L.qdense + (uint64_t(L.nq_pad) * hq + 4 * kQTile) * kMaxHeadDim * 2 + 255) & ~uint64_t(255);
-  L.bytes = (L.chunk_stats + uint64_t(kMaxRowChunks) * hq * L.nq_pad * 8 + 255) & ~uint64_t(255);
+  L.bytes = (L.chunk_stats + uint64_t(max_row_chunks(uint64_t(hq) * std::max(1u, L.nq_pad))) * hq * L.nq_pad * 8 + 255) & ~uint64_t(255);
   return L;
 }
 
@@ -882,16 +905,28 @@ constexpr uint32_t kRowChunkTarget = 6;  // rowstats workgroups per resident slo
 // 3.445-3.446 ms same box; 3 ranges 3.444-3.446, 4 ranges 3.449).
 constexpr uint32_t kColSplitTarget = 4;
 
-uint32_t col_splits(uint32_t units, int cus) {
+// A range of fewer than four units costs more in re-read keys than it saves
+// (K is read once a range: 64 queries of 16383 keys, 32 heads over 8, 54 us a
+// call at 4 ranges of one unit, 47 at one), unless the key blocks alone leave
+// CUs without a workgroup (2000 keys: 31 -> 29 us at 4).
+uint32_t col_splits(uint32_t groups, uint32_t units, int cus) {
   const uint32_t slots = 3u * uint32_t(cus);
-  const uint32_t k = units ? (kColSplitTarget * slots + units - 1) / units : 1u;
-  return std::max(1u, std::min(kMaxColSplits, k));
+  const uint32_t fill = std::min(units, uint32_t(cus) / std::max(1u, groups));
+  const uint32_t even = std::min(units / 4, groups ? (kColSplitTarget * slots + groups - 1) / groups : 1u);
+  return std::max(1u, std::min(kMaxColSplits, std::max(fill, even)));
 }
 
-uint32_t row_chunks(uint32_t units, int cus, uint32_t per_cu) {
+// More than 8 ranges, where the statistics' scratch allows it (`most`), only
+// to give every CU a workgroup, or where a range keeps 32 key blocks. us a call
+// at 8 / 16 / 32 / 64 ranges, 32 heads over 8: 64 queries of 16383 keys 81 /
+// 61 / 51 / 52; 200 of 4000 43 / 44 / 53 / 71; 500 of 16000 160 / 150 / 162 /
+// 201; 1500 of 16000 (16 over 8) 143 / 157 / 194 / 268.
+uint32_t row_chunks(uint32_t groups, uint32_t key_blocks, int cus, uint32_t per_cu, uint32_t most) {
   const uint32_t slots = per_cu * uint32_t(cus);  // rowstats workgroups resident per CU
-  const uint32_t k = units ? (kRowChunkTarget * slots + units - 1) / units : 1u;
-  return std::max(1u, std::min(kMaxRowChunks, k));
+  const uint32_t fill = uint32_t(cus) / std::max(1u, groups);
+  const uint32_t even = std::min(groups ? (kRowChunkTarget * slots + groups - 1) / groups : 1u,
+                                 std::max(8u, key_blocks / 32));
+  return std::max(1u, std::min(most, std::max(fill, even)));
 }
 
 // Sets the launch's key ranges in `a`.
@@ -910,14 +945,18 @@ int launch_mfma_ks(SqArgs& a, int cus, hipStream_t stream) {
   const uint32_t tpw = a.groups <= 4 ? 4u : a.groups <= 8 ? 2u : 1u;
   const uint64_t tgroups = (ntiles + tpw - 1) / tpw;
   const int waves = tpw == 4 ? ((KS == 4 || a.groups >= 3) ? 2 : 3) : tpw == 2 ? 2 : (a.groups > 8 && KS == 4) ? 2 : 3;
-  a.row_chunks = row_chunks(uint32_t(tgroups * a.hkv), cus, uint32_t(waves));
+  a.row_chunks = row_chunks(uint32_t(tgroups * a.hkv), (a.nk + kKeyBlock1 - 1) / kKeyBlock1, cus, uint32_t(waves),
+                            max_row_chunks(uint64_t(a.hq) * a.nq_pad));
   // one-dimensional grids (the kv head fastest): every launch within 2^32 threads
   CBK_REQUIRE(tgroups * a.hkv * a.row_chunks * kThreads < (uint64_t(1) << 32) &&
                   kblocks * a.hkv * kMaxColSplits * kThreads < (uint64_t(1) << 32) &&
                   uint64_t(a.hq) * a.nq_pad < (uint64_t(1) << 32),
               "sparse_q: %llu query tiles x %llu key blocks x %u kv heads exceed one launch",
               (unsigned long long)ntiles, (unsigned long long)kblocks, a.hkv);
-  a.col_splits = col_splits(uint32_t(kblocks * a.hkv), cus);
+  // column units of a key block that every query sees (chunks of 4 heads, or
+  // four (tile, head) rows)
+  const uint64_t units = ntiles * a.groups / kHeadChunk + (ntiles * a.groups % kHeadChunk != 0);
+  a.col_splits = col_splits(uint32_t(kblocks * a.hkv), uint32_t(units), cus);
   // units of four (tile, head) rows address a KV head's statistics with
   // per-lane 32-bit byte offsets
   CBK_REQUIRE(a.groups % kHeadChunk == 0 || uint64_t(a.groups) * a.nq_pad * 8 < (uint64_t(1) << 31),
@@ -979,7 +1018,7 @@ int launch_mfma(SqArgs& a, int ksteps, hipStream_t stream) {
 }  // namespace
 
 void launch_sq_merge(const SqArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL(sq_merge_kernel, dim3((a.hq * a.nq_pad + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, a);
+  hipLaunchKernelGGL(sq_merge_kernel, dim3((a.hq * a.nq_pad + 63) / 64), dim3(kThreads), 0, stream, a);
 }
 
 }  // namespace cbk

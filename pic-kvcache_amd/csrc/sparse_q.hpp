@@ -70,8 +70,13 @@ int launch_sq_f32(SqArgs& a, hipStream_t stream);
 // Merges the key ranges' statistics of every (head, query) row (row_chunks > 1).
 void launch_sq_merge(const SqArgs& a, hipStream_t stream);
 
-// Key ranges a (query tile, kv head) of the row pass may be split into.
-constexpr uint32_t kMaxRowChunks = 8;
+// Key ranges a (query tile, kv head) of the row pass may be split into, for
+// `rows` = hq * nq_pad statistics: few rows leave most of the chip without a
+// tile, and their ranges' statistics are small (16 MB at most past 8 ranges).
+inline uint32_t max_row_chunks(uint64_t rows) {
+  const uint64_t fit = (uint64_t(16) << 20) / (rows * sizeof(float2));
+  return fit < 8 ? 8u : fit > 64 ? 64u : uint32_t(fit);
+}
 // Query ranges a (key block, kv head) of the column pass may be split into.
 constexpr uint32_t kMaxColSplits = 4;
 

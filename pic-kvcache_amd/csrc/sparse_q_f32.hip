@@ -328,7 +328,7 @@ int launch_sq_f32(SqArgs& a, hipStream_t stream) {
   const uint64_t rows = uint64_t(a.nq) * a.groups;
   CBK_REQUIRE(rows < (uint64_t(1) << 31), "sparse_q: %llu rows per KV head exceed one launch", (unsigned long long)rows);
   const uint64_t u1 = (rows + kTile - 1) / kTile * a.hkv, u2 = (uint64_t(a.nk) + kTile - 1) / kTile * a.hkv;
-  a.row_chunks = ranges(u1, cus, kMaxRowChunks);
+  a.row_chunks = ranges(u1, cus, max_row_chunks(uint64_t(a.hq) * a.nq_pad));
   a.col_splits = ranges(u2, cus, kMaxColSplits);
   CBK_REQUIRE(u1 * a.row_chunks * kThreads < (uint64_t(1) << 32) && u2 * a.col_splits * kThreads < (uint64_t(1) << 32),
               "sparse_q: %llu rows x %u keys exceed one launch", (unsigned long long)rows, a.nk);

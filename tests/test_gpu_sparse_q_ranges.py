@@ -67,3 +67,26 @@ def test_f32_unaligned_views():
     _, want = S.sparse_q_full_scores(q.to(DEV), k.to(DEV), None, pos.to(DEV), 0.125, want_full=True)
     _, got = S.sparse_q_full_scores(off(q), off(k), None, pos.to(DEV), 0.125, want_full=True)
     assert torch.equal(got, want)
+
+
+# few rows over many keys: up to 64 key ranges (more than the merge's batch of
+# loads per wave, ranges without a block, and key counts around a block), column
+# units in one to four ranges; entries in {-1, 0, 1} / 8, whose dot products
+# are exact in the input type
+@pytest.mark.parametrize("nq,nk,hq,hkv,d,dtype", [
+    (1, 16385, 1, 1, 64, torch.bfloat16), (64, 9001, 4, 1, 128, torch.bfloat16), (17, 4095, 8, 1, 64, torch.float16),
+    (64, 700, 3, 1, 128, torch.float16), (200, 2050, 2, 2, 128, torch.bfloat16), (33, 6000, 16, 1, 64, torch.bfloat16),
+])
+def test_16_bit_matches_float64(nq, nk, hq, hkv, d, dtype):
+    g = torch.Generator().manual_seed(nq + nk)
+    q, k = ((torch.randint(-1, 2, (n, h, d), generator=g) / 8).to(dtype) for n, h in ((nq, hq), (nk, hkv)))
+    pos = torch.randint(0, nk, (nq,), generator=g).sort().values
+    pos[-1] = nk - 1
+    rows = torch.arange(nq)
+    _, full = S.sparse_q_full_scores(q.to(DEV), k.to(DEV), None, pos.to(DEV), 1.0, want_full=True)
+    want, size = _f64(q, k, rows, pos, 1.0)
+    # exact logits: the float32 exponentials and sums of positive terms only
+    bound = (nk + nq * hq + 24 + 4 * size) * 2.0 ** -24
+    err = np.abs(full.cpu().numpy() - want) / np.maximum(want, 1e-300)
+    print(f"largest error / bound {err.max() / bound:.3f}", flush=True)
+    assert err.max() <= bound
