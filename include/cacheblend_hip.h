@@ -432,6 +432,18 @@ int cbk_sparse_q_scores(const void* q_dev, int64_t q_row_stride_elems, const int
 int cbk_dilate(const uint8_t* gap_dev, int64_t n, int64_t radius, uint8_t* forced_dev,
                cbk_stream_t stream);
 
+/*
+ * The Sparse-Q queries and forced tokens of a gap mask (cacheblend_vllm/
+ * ascend.py:652-671): with gaps, rows = the gaps' indices in order and forced =
+ * the gaps dilated by `radius`; without any, rows = the last min(tail, n)
+ * tokens (all n for a tail of 0, as Python's x[-0:]) and forced = those.
+ * rows_dev holds up to n entries, counts_dev cbk_sparse_q_rows_counts(n) int64
+ * words, whose first becomes the number of gaps; n > 0.
+ */
+size_t cbk_sparse_q_rows_counts(int64_t n);
+int cbk_sparse_q_rows(const uint8_t* gap_dev, int64_t n, int64_t tail, int64_t radius, uint8_t* forced_dev,
+                      int64_t* rows_dev, int64_t* counts_dev, cbk_stream_t stream);
+
 /* ------------------------------------------------ token-range matcher
  * Host code (no GPU calls): the scheduler-side lookup that finds stored
  * chunks at any offset of a prompt. Tokens are int64; a chunk's hash is

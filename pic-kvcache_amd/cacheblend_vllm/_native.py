@@ -106,6 +106,8 @@ _SIGNATURES = {
         ],
     ),
     "cbk_dilate": (ctypes.c_int, [c_vp, c_i64, c_i64, c_vp, c_vp]),
+    "cbk_sparse_q_rows_counts": (ctypes.c_size_t, [c_i64]),
+    "cbk_sparse_q_rows": (ctypes.c_int, [c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp]),
     "cbk_blend_assemble": (
         ctypes.c_int,
         [

@@ -321,6 +321,26 @@ def sparse_q_query_rows(query_mask: torch.Tensor, has_gap: bool, gap_count: int,
     return torch.nonzero_static(query_mask, size=n_rows).flatten()
 
 
+def sparse_q_rows(gap_mask: torch.Tensor, tail_query_tokens: int, radius: int):
+    """``(rows, forced_mask, gap_count)`` of a bool device mask: what
+    ``sparse_q_masks`` and ``sparse_q_query_rows`` give, in two launches and
+    one host read (``cbk_sparse_q_rows``)."""
+    n = int(gap_mask.shape[0])
+    dev = gap_mask.device
+    gap = _mask_u8(gap_mask, n, "gap_mask")
+    lib = _native.load()
+    forced = torch.empty(n, dtype=torch.bool, device=dev)
+    # the counts behind the rows: one allocation
+    rows = torch.empty(n + lib.cbk_sparse_q_rows_counts(n), dtype=torch.long, device=dev)
+    counts = rows[n:]
+    rc = lib.cbk_sparse_q_rows(gap.data_ptr(), n, tail_query_tokens, radius, forced.data_ptr(), rows.data_ptr(),
+                               counts.data_ptr(), _native.stream_handle(dev))
+    _native.check(rc, "sparse_q_rows")
+    gap_count = int(counts[0].item())
+    tail = min(tail_query_tokens, n) if tail_query_tokens else n
+    return rows[: gap_count or tail], forced, gap_count
+
+
 @dataclass
 class CheckLayerSelection:
     """What the check layer's selection block produces (ascend.py:529-531)."""
@@ -385,13 +405,16 @@ class BlendSelector:
         radius = self.config.overflow_blocks * self.block_size
         if gap_mask.dtype != torch.bool:
             gap_mask = gap_mask != 0
-        # the one host read before the scores; count_nonzero, as the masks
-        # treat any nonzero entry as set (a sum would overcount 2s and size
-        # the query compaction past the set rows)
-        gap_count = int(gap_mask.count_nonzero().item())
+        # one host read before the scores: the query count sizes their launches
         tail = self.config.tail_query_tokens
-        query_mask, forced, has_gap = sparse_q_masks(gap_mask, tail, radius, gap_count=gap_count)
-        sparse = sparse_q_query_rows(query_mask, has_gap, gap_count, tail)
+        if gap_mask.is_cuda and gap_mask.ndim == 1 and gap_mask.shape[0] and radius <= _native.MAX_DILATION_RADIUS:
+            sparse, forced, gap_count = sparse_q_rows(gap_mask, tail, radius)
+            has_gap = gap_count > 0
+        else:
+            # count_nonzero, as the masks treat any nonzero entry as set
+            gap_count = int(gap_mask.count_nonzero().item())
+            query_mask, forced, has_gap = sparse_q_masks(gap_mask, tail, radius, gap_count=gap_count)
+            sparse = sparse_q_query_rows(query_mask, has_gap, gap_count, tail)
         scores, _ = sparse_q_full_scores(query, key, sparse, absolute_indices, scale,
                                          out_index=absolute_indices)
         stats = {

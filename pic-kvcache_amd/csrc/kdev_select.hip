@@ -1422,6 +1422,113 @@ __global__ __launch_bounds__(256) void dilate_kernel(const uint8_t* gap, uint32_
   }
 }
 
+// ---------------------------------------------------- Sparse-Q query rows
+// Two small launches in place of a count, two clones, a dilation, an "or" and
+// a four-kernel compaction: latency-bound, about 3 us each (16383 tokens),
+// against ten launches and 45 us between the caller's read of the count and
+// the scores.
+//   masks  forced = gap, dilated by r; the tile's gap count
+//   rows   the earlier tiles' counts give the tile's place: the gaps in index
+//          order; without any gap the last `tail` tokens, which are then
+//          forced too
+
+constexpr int kRowItems = 8;
+constexpr int kRowTile = 256 * kRowItems;
+
+// 8 flags from `i0` on, bit e for token i0 + e; one load where it is aligned
+__device__ __forceinline__ uint32_t flag_bits8(const uint8_t* gap, uint32_t i0, uint32_t n) {
+  uint32_t bits = 0;
+  if (i0 + 8 <= n && (reinterpret_cast<uintptr_t>(gap + i0) & 7) == 0) {
+    const uint64_t w = *reinterpret_cast<const uint64_t*>(gap + i0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bits |= ((w >> (8 * e)) & 0xFFull) ? (1u << e) : 0u;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (i0 + e < n && gap[i0 + e]) bits |= 1u << e;
+  }
+  return bits;
+}
+
+__global__ __launch_bounds__(256) void sparse_q_masks_kernel(const uint8_t* gap, uint32_t n, int32_t r,
+                                                             uint8_t* forced, int64_t* counts) {
+  extern __shared__ uint32_t win[];  // kRowTile + 2r prefix counts of gaps, r > 0
+  __shared__ uint32_t scan[8];
+  const uint32_t tile0 = blockIdx.x * kRowTile;
+  const uint32_t i0 = tile0 + threadIdx.x * kRowItems;
+  if (r > 0) {
+    const uint32_t W = kRowTile + 2 * r;
+    const uint32_t per = (W + 255) / 256;
+    const uint32_t beg = threadIdx.x * per;
+    const uint32_t end = min(W, beg + per);
+    uint32_t local = 0;
+    for (uint32_t w = beg; w < end; ++w) {
+      const int64_t g = int64_t(tile0) - r + w;
+      local += (g >= 0 && g < int64_t(n) && gap[g]) ? 1u : 0u;
+      win[w] = local;
+    }
+    uint32_t total;
+    const uint32_t excl = block_exclusive_scan<256>(local, scan, &total);
+    for (uint32_t w = beg; w < end; ++w) win[w] += excl;
+    __syncthreads();
+  }
+  const uint32_t bits = i0 < n ? flag_bits8(gap, i0, n) : 0u;
+  uint64_t out = 0;
+#pragma unroll
+  for (int e = 0; e < kRowItems; ++e) {
+    bool f = (bits >> e) & 1u;
+    if (r > 0 && i0 + e < n) {
+      const uint32_t k = i0 + e - tile0 + r;  // the token's place in the window
+      f = win[k + r] > (k >= uint32_t(r) + 1 ? win[k - r - 1] : 0u);
+    }
+    out |= f ? (1ull << (8 * e)) : 0ull;
+  }
+  if (i0 + kRowItems <= n && (reinterpret_cast<uintptr_t>(forced + i0) & 7) == 0) {
+    *reinterpret_cast<uint64_t*>(forced + i0) = out;
+  } else {
+#pragma unroll
+    for (int e = 0; e < kRowItems; ++e)
+      if (i0 + e < n) forced[i0 + e] = uint8_t(out >> (8 * e));
+  }
+  uint32_t tile_gaps;
+  block_exclusive_scan<256>(__popc(bits), scan, &tile_gaps);
+  if (threadIdx.x == 0) counts[1 + blockIdx.x] = int64_t(tile_gaps);
+}
+
+__global__ __launch_bounds__(256) void sparse_q_rows_kernel(const uint8_t* gap, uint32_t n, uint32_t tail,
+                                                            uint8_t* forced, int64_t* rows, int64_t* counts) {
+  __shared__ uint32_t scan[8];
+  const uint32_t i0 = blockIdx.x * kRowTile + threadIdx.x * kRowItems;
+  uint32_t before = 0, all = 0;
+  for (uint32_t t = threadIdx.x; t < gridDim.x; t += 256) {
+    const uint32_t c = uint32_t(counts[1 + t]);
+    all += c;
+    before += t < blockIdx.x ? c : 0u;
+  }
+  uint32_t total, place;
+  block_exclusive_scan<256>(all, scan, &total);
+  block_exclusive_scan<256>(before, scan, &place);
+  if (blockIdx.x == 0 && threadIdx.x == 0) counts[0] = int64_t(total);
+  if (total == 0) {
+    const uint32_t first = n - tail;
+#pragma unroll
+    for (int e = 0; e < kRowItems; ++e) {
+      const uint32_t i = i0 + e;
+      if (i >= first && i < n) {
+        rows[i - first] = int64_t(i);
+        forced[i] = 1;
+      }
+    }
+    return;
+  }
+  const uint32_t bits = i0 < n ? flag_bits8(gap, i0, n) : 0u;
+  uint32_t tile_gaps;
+  uint32_t at = place + block_exclusive_scan<256>(__popc(bits), scan, &tile_gaps);
+#pragma unroll
+  for (int e = 0; e < kRowItems; ++e)
+    if ((bits >> e) & 1u) rows[at++] = int64_t(i0 + e);
+}
+
 }  // namespace
 
 // ------------------------------------------------ allocation-free selection
@@ -1581,6 +1688,29 @@ int cbk_dilate(const uint8_t* gap_dev, int64_t n, int64_t radius, uint8_t* force
   hipLaunchKernelGGL(cbk::dilate_kernel, dim3(grid), dim3(256), lds, static_cast<hipStream_t>(stream),
                      gap_dev, uint32_t(n), int32_t(radius), forced_dev);
   return cbk::launch_status("dilate");
+}
+
+size_t cbk_sparse_q_rows_counts(int64_t n) {
+  return n <= 0 ? 1 : size_t(1 + (n + cbk::kRowTile - 1) / cbk::kRowTile);
+}
+
+int cbk_sparse_q_rows(const uint8_t* gap_dev, int64_t n, int64_t tail, int64_t radius, uint8_t* forced_dev,
+                      int64_t* rows_dev, int64_t* counts_dev, cbk_stream_t stream) {
+  cbk::clear_error();
+  CBK_REQUIRE(n > 0 && n < (int64_t(1) << 31), "n out of range");
+  CBK_REQUIRE(tail >= 0, "tail must be non-negative");
+  CBK_REQUIRE(radius >= 0 && radius <= CBK_MAX_DILATION_RADIUS,
+              "dilation radius %lld outside [0, %d]", (long long)radius, CBK_MAX_DILATION_RADIUS);
+  CBK_REQUIRE(gap_dev && forced_dev && rows_dev && counts_dev, "NULL pointer");
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const uint32_t grid = uint32_t((n + cbk::kRowTile - 1) / cbk::kRowTile);
+  const size_t lds = radius > 0 ? (cbk::kRowTile + 2 * size_t(radius)) * sizeof(uint32_t) : 0;
+  const uint32_t last = uint32_t(tail == 0 || tail > n ? n : tail);
+  hipLaunchKernelGGL(cbk::sparse_q_masks_kernel, dim3(grid), dim3(256), lds, s, gap_dev, uint32_t(n),
+                     int32_t(radius), forced_dev, counts_dev);
+  hipLaunchKernelGGL(cbk::sparse_q_rows_kernel, dim3(grid), dim3(256), 0, s, gap_dev, uint32_t(n), last, forced_dev,
+                     rows_dev, counts_dev);
+  return cbk::launch_status("sparse_q rows");
 }
 
 }  // extern "C"
