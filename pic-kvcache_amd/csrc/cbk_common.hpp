@@ -150,42 +150,41 @@ __device__ __forceinline__ float row16_reduce(float v, F op) {
   return v;
 }
 
-// Inclusive prefix sum over the 64 lanes of a wavefront.
+// Inclusive prefix sum over the 64 lanes of a wavefront, by DPP: shifts within
+// the rows of 16 lanes, then the rows' totals broadcast to the rows after.
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    uint32_t o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
-  }
+#define CBK_DPP_SCAN(ctrl, rows) v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), ctrl, rows, 0xf, false))
+  CBK_DPP_SCAN(0x111, 0xf);  // row_shr 1, 2, 4, 8
+  CBK_DPP_SCAN(0x112, 0xf);
+  CBK_DPP_SCAN(0x114, 0xf);
+  CBK_DPP_SCAN(0x118, 0xf);
+  CBK_DPP_SCAN(0x142, 0xa);  // row_bcast 15: into rows 1 and 3
+  CBK_DPP_SCAN(0x143, 0xc);  // row_bcast 31: into rows 2 and 3
+#undef CBK_DPP_SCAN
   return v;
 }
 
 // Exclusive block-wide scan for a block of NT threads (NT multiple of 64).
-// `lds` needs NT/64 + 1 uint32 slots. Returns the exclusive prefix of `v`
+// `lds` needs NT/64 uint32 slots. Returns the exclusive prefix of `v`
 // and writes the block total to *total.
 template <int NT>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* lds, uint32_t* total) {
   constexpr int NW = NT / 64;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  uint32_t inc = wave_inclusive_scan(v);
+  const uint32_t inc = wave_inclusive_scan(v);
   if (lane == 63) lds[wave] = inc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t run = 0;
-    for (int w = 0; w < NW; ++w) {
-      uint32_t t = lds[w];
-      lds[w] = run;
-      run += t;
-    }
-    lds[NW] = run;
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const uint32_t t = lds[w];
+    before += w < wave ? t : 0u;
+    all += t;
   }
   __syncthreads();
-  uint32_t result = lds[wave] + inc - v;
-  *total = lds[NW];
-  __syncthreads();
-  return result;
+  *total = all;
+  return before + inc - v;
 }
 
 // bf16 / f16 / f32 element loads widened to float.

@@ -16,6 +16,9 @@
 //   tiecount per-tile counts of key == T and of sure picks; last block:
 //           tie offsets, output offsets, total
 //   write   per-tile ordered compaction of selected indices
+// One launch does all of it where the device holds every tile's block at once
+// (sel_onepass_kernel), and one block where that holds every token
+// (sel_block_kernel).
 // (the fused K-deviation launch clears the counters in its first block, so
 // the zero launch is skipped there)
 // Every tile is 2048 consecutive tokens (8 per thread), so tile order is
@@ -1253,6 +1256,169 @@ __global__ __launch_bounds__(NT) void sel_onepass_kernel(const SelArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------
+// Selections of one block's tokens (NT * ITEMS at most): the whole select in
+// registers and LDS, no counters, barriers or candidate lists in memory. The
+// k-th key's three digits (12, 12 and 8 bits) by LDS histograms of the keys
+// that share the digits before, ties in index order by a scan.
+// Latency-bound: a launch, one load and a few dozen LDS steps.
+// ---------------------------------------------------------------------
+
+// The digit (of NBINS) holding the k-th largest of the histogram in LDS, and
+// k's rank inside it. Ends with a barrier.
+template <int NT, int NBINS>
+__device__ __forceinline__ void block_digit(const uint32_t* hist, uint32_t k, uint32_t* scan, uint32_t* out) {
+  constexpr int PER = NBINS > NT ? NBINS / NT : 1;
+  const int top = NBINS - PER * int(threadIdx.x + 1);  // this thread's lowest bin
+  uint32_t c[PER], s = 0;
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    c[p] = top >= 0 ? hist[top + p] : 0u;
+    s += c[p];
+  }
+  uint32_t total;
+  uint32_t run = block_exclusive_scan<NT>(s, scan, &total);  // larger keys than this thread's
+  if (run < k && k <= run + s) {
+#pragma unroll
+    for (int p = PER - 1; p >= 0; --p) {
+      if (run < k && k <= run + c[p]) {
+        out[0] = uint32_t(top + p);
+        out[1] = k - run;
+      }
+      run += c[p];
+    }
+  }
+  __syncthreads();
+}
+
+template <int NT, int ITEMS>
+__global__ __launch_bounds__(NT) void sel_block_kernel(const SelArgs a) {
+  extern __shared__ uint32_t window[];  // NT * ITEMS prefix counts of gaps, r > 0
+  __shared__ __attribute__((aligned(16))) uint32_t hist[4096];
+  __shared__ uint32_t scan[NT / 64], scan2[NT / 64], digit[2];
+  const uint32_t i0 = threadIdx.x * ITEMS;
+  const int r = a.radius;
+  float sc[ITEMS];
+  uint32_t gap = 0, base = 0;  // bit e: token i0 + e
+  if (a.vec_ok && i0 + ITEMS <= a.n) {
+#pragma unroll
+    for (int q = 0; q < ITEMS / 4; ++q) {
+      const float4 v = *reinterpret_cast<const float4*>(a.scores + i0 + 4 * q);
+      sc[4 * q] = v.x; sc[4 * q + 1] = v.y; sc[4 * q + 2] = v.z; sc[4 * q + 3] = v.w;
+    }
+#pragma unroll
+    for (int q = 0; q < ITEMS / 8; ++q) {
+      const uint64_t g8 = *reinterpret_cast<const uint64_t*>(a.gap + i0 + 8 * q);
+      const uint64_t f8 = a.forced ? *reinterpret_cast<const uint64_t*>(a.forced + i0 + 8 * q) : 0ull;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        gap |= ((g8 >> (8 * e)) & 0xFFull) ? 1u << (8 * q + e) : 0u;
+        base |= ((f8 >> (8 * e)) & 0xFFull) ? 1u << (8 * q + e) : 0u;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e) {
+      const uint32_t i = i0 + e;
+      const bool in = i < a.n;
+      sc[e] = in ? a.scores[i] : 0.f;
+      gap |= in && a.gap[i] ? 1u << e : 0u;
+      base |= in && a.forced && a.forced[i] ? 1u << e : 0u;
+    }
+  }
+  base |= gap;
+  const uint32_t valid = i0 >= a.n ? 0u : a.n - i0 >= uint32_t(ITEMS) ? (1u << ITEMS) - 1u : (1u << (a.n - i0)) - 1u;
+  if (r > 0) {
+    // prefix counts of gaps (tokens 0 .. i), a thread's NT words apart: the
+    // lanes of an access read consecutive words (16 tokens a thread side by
+    // side: 10 us more at 16384 tokens)
+    auto at = [](uint32_t i) { return (i % ITEMS) * NT + i / ITEMS; };
+    uint32_t total;
+    const uint32_t excl = block_exclusive_scan<NT>(__popc(gap), scan, &total);
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e) window[at(i0 + e)] = excl + __popc(gap & ((2u << e) - 1u));
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e) {
+      const uint32_t i = i0 + e;
+      if (i < a.n) {
+        const uint32_t hi = window[at(min(i + uint32_t(r), a.n - 1))];
+        const uint32_t lo = i > uint32_t(r) ? window[at(i - r - 1)] : 0u;
+        base |= hi > lo ? 1u << e : 0u;
+      }
+    }
+  }
+  uint32_t key[ITEMS];
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e) key[e] = (base >> e) & 1u ? kKeyNegInf : order_key(sc[e]);
+#pragma unroll
+  for (int q = 0; q < 1024 / NT; ++q) reinterpret_cast<uint4*>(hist)[threadIdx.x + q * NT] = make_uint4(0u, 0u, 0u, 0u);
+  // gaps in the low, base tokens in the high half (n <= 16384)
+  uint32_t counts;
+  block_exclusive_scan<NT>(__popc(gap) + (__popc(base) << 16), scan2, &counts);
+  const uint32_t gaps = counts & 0xFFFFu, bases = counts >> 16;
+  // budget: int(cached * ratio) as Python computes it, then [1, available]
+  int64_t topk = 0;
+  const int64_t cached = int64_t(a.n) - gaps, available = int64_t(a.n) - bases;
+  if (cached && available) {
+    topk = int64_t(double(cached) * a.ratio);
+    topk = topk < 1 ? 1 : topk;
+    topk = topk > available ? available : topk;
+  }
+  uint32_t write = base;
+  if (topk > 0) {  // uniform
+    // first digit; the base tokens' bin is added as a whole
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e)
+      if ((valid & ~base) >> e & 1u) atomicAdd(&hist[key[e] >> 20], 1u);
+    if (threadIdx.x == 0 && bases) atomicAdd(&hist[kKeyNegInf >> 20], bases);
+    __syncthreads();
+    block_digit<NT, 4096>(hist, uint32_t(topk), scan, digit);
+    uint32_t prefix = digit[0], want = digit[1];
+#pragma unroll
+    for (int q = 0; q < 1024 / NT; ++q)
+      reinterpret_cast<uint4*>(hist)[threadIdx.x + q * NT] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e)
+      if ((valid >> e & 1u) && (key[e] >> 20) == prefix) atomicAdd(&hist[(key[e] >> 8) & 0xFFFu], 1u);
+    __syncthreads();
+    block_digit<NT, 4096>(hist, want, scan, digit);
+    prefix = (prefix << 12) | digit[0];
+    want = digit[1];
+    if (threadIdx.x < 64) reinterpret_cast<uint4*>(hist)[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e)
+      if ((valid >> e & 1u) && (key[e] >> 8) == prefix) atomicAdd(&hist[key[e] & 0xFFu], 1u);
+    __syncthreads();
+    block_digit<NT, 256>(hist, want, scan, digit);
+    const uint32_t T = (prefix << 8) | digit[0];
+    want = digit[1];
+    uint32_t ties = 0;
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e) {
+      if (!(valid >> e & 1u)) continue;
+      if (key[e] > T) write |= 1u << e;
+      if (key[e] == T) ties |= 1u << e;
+    }
+    uint32_t total;
+    uint32_t rank = block_exclusive_scan<NT>(__popc(ties), scan, &total);
+#pragma unroll
+    for (int e = 0; e < ITEMS; ++e)
+      if (ties >> e & 1u) {
+        if (rank < want) write |= 1u << e;
+        ++rank;
+      }
+  }
+  uint32_t total;
+  uint32_t pos = block_exclusive_scan<NT>(__popc(write), scan2, &total);
+  if (threadIdx.x == 0) *a.out_count = int64_t(total);
+#pragma unroll
+  for (int e = 0; e < ITEMS; ++e)
+    if (write >> e & 1u) a.out_idx[pos++] = int64_t(i0 + e);
+}
+
 __global__ void write_zero_count_kernel(int64_t* out_count) { *out_count = 0; }
 
 int check_select(const float* scores, const uint8_t* gap, int64_t n, int64_t radius, double ratio,
@@ -1334,6 +1500,25 @@ int launch_onepass(const SelArgs& a, int64_t n, int64_t radius, hipStream_t stre
   return launch_status("select (one launch)");
 }
 
+// Tokens that the one-block select takes, 8 or 16 a thread. us a select,
+// one-launch form before -> one block: 1537 tokens 15.5 -> 8.0, 8192 17.5 -> 8.4,
+// 16384 17.6 -> 13.0; with a dilation of 16 18.5 -> 9.1, 18.6 -> 10.3, 18.9 ->
+// 16.2 (past that one CU's LDS passes take longer than the grid's barriers).
+constexpr int64_t kBlockTokens = 16384;
+
+template <int NT, int ITEMS>
+int launch_block_t(const SelArgs& a, int64_t radius, hipStream_t stream) {
+  const size_t lds = radius > 0 ? size_t(NT) * ITEMS * sizeof(uint32_t) : 0;
+  hipLaunchKernelGGL((sel_block_kernel<NT, ITEMS>), dim3(1), dim3(NT), lds, stream, a);
+  return launch_status("select (one block)");
+}
+
+int launch_block_select(const SelArgs& a, int64_t n, int64_t radius, hipStream_t stream) {
+  if (n <= 2048) return launch_block_t<256, 8>(a, radius, stream);
+  if (n <= 8192) return launch_block_t<1024, 8>(a, radius, stream);
+  return launch_block_t<1024, 16>(a, radius, stream);
+}
+
 // header_zeroed: an earlier launch on the stream cleared the kHeader counter
 // words (the fused K-deviation launch does). flags: CBK_SELECT_* bits.
 int launch_select(const float* scores, const uint8_t* gap, const uint8_t* forced, int64_t n,
@@ -1372,6 +1557,9 @@ int launch_select(const float* scores, const uint8_t* gap, const uint8_t* forced
   const bool give_up = (flags & CBK_SELECT_TEST_GIVE_UP) != 0;
   a.spin_limit = give_up ? 0u : kBarrierSpins;
   a.bar_extra = give_up ? 1u : 0u;
+  // one block's tokens: everything in its LDS (CBK_SELECT_TEST_GIVE_UP asks
+  // for the grid barrier, CBK_SELECT_MULTI_LAUNCH for the launches below)
+  if (flags == 0 && n <= kBlockTokens) return launch_block_select(a, n, radius, stream);
   if (!header_zeroed) hipLaunchKernelGGL(sel_zero_kernel, dim3(1), dim3(kSelThreads), 0, stream, a.ws);
   // one launch when every tile's block can be resident at once
   if ((flags & CBK_SELECT_MULTI_LAUNCH) == 0) {
