@@ -171,14 +171,21 @@ class PagedBlendLoader:
             )
         src, old, relocate = build_source_map(plan)
         self._relocate = relocate
-        self._src_map = torch.from_numpy(src).to(self.device)
-        self._old_pos = torch.from_numpy(old).to(self.device) if old.size else None
         num_slots = key.shape[0] * block_size
-        if self.slot_mapping.device.type == "cpu" and self.slot_mapping.numel():
-            lo, hi = int(self.slot_mapping.min()), int(self.slot_mapping.max())
+        slots = self.slot_mapping
+        if slots.device.type == "cpu" and slots.numel():
+            lo, hi = int(slots.min()), int(slots.max())
             if lo < 0 or hi >= num_slots:
                 raise IndexError(f"slot_mapping holds slots in [{lo}, {hi}], outside [0, {num_slots})")
-        self._slots = self.slot_mapping.to(device=self.device, dtype=torch.long).contiguous()
+        self._load_stream = None
+        self._copy_stream: torch.cuda.Stream | None = None
+        if config.event_pipeline:
+            self._load_stream = load_stream or side_stream(LOAD, self.device)
+            self._copy_stream = copy_stream or side_stream(COPY, self.device)
+        # the Load stream's tables; the serving streams that may read the slots
+        self._tables_event: torch.cuda.Event | None = None
+        self._slots_ready: set[int] = set()
+        self._upload_tables(src, old, slots)
         self._buffers: dict[int, torch.Tensor] = {}
         self._events: dict[int, torch.cuda.Event] = {}
         self._reuse_events: dict[int, torch.cuda.Event] = {}
@@ -195,7 +202,6 @@ class PagedBlendLoader:
         self._ring_layers = layers
         # the last GPU event after which this loader reads no host memory
         self._host_reads: torch.cuda.Event | None = None
-        self._copy_stream: torch.cuda.Stream | None = None
         self._descs: dict[int, _native.KVDesc] = {}
         self._zero_copy = zero_copy
         self._max_workgroups = max_workgroups
@@ -203,14 +209,6 @@ class PagedBlendLoader:
         self._ptr_host: torch.Tensor | None = None  # [layers, chunks, 2] pinned
         self._ptr_dev: torch.Tensor | None = None
         self._zc_layers: set[int] = set()
-        self._load_stream = None
-        if config.event_pipeline:
-            self._load_stream = load_stream or side_stream(LOAD, self.device)
-            self._copy_stream = copy_stream or side_stream(COPY, self.device)
-            # tables made on the current stream are read on the Load stream
-            for table in (self._src_map, self._old_pos, self._slots):
-                if table is not None:
-                    table.record_stream(self._load_stream)
         if tracer is not None and tracer.enabled:
             tracer.emit(
                 "loader_initialized",
@@ -223,6 +221,47 @@ class PagedBlendLoader:
             )
 
     # ------------------------------------------------------------ helpers
+
+    def _upload_tables(self, src: np.ndarray, old: np.ndarray, slots: torch.Tensor) -> None:
+        """The slots, the source map and the old positions on the device. With
+        a Load stream they go up on it in one copy from page-locked memory: a
+        copy on the serving stream would wait there (and, from pageable
+        memory, make the host wait) for the work of the requests before, and
+        with it this request's first DMA."""
+        if self._load_stream is None or slots.device.type != "cpu":
+            self._src_map = torch.from_numpy(src).to(self.device)
+            self._old_pos = torch.from_numpy(old).to(self.device) if old.size else None
+            self._slots = slots.to(device=self.device, dtype=torch.long).contiguous()
+            if self._load_stream is not None:
+                for table in (self._src_map, self._old_pos, self._slots):
+                    if table is not None:
+                        table.record_stream(self._load_stream)
+            return
+        n, hits = src.size, old.size
+        host = torch.empty(2 * n + n + hits, dtype=torch.int32, pin_memory=True)
+        host[: 2 * n].view(torch.long).copy_(slots)
+        flat = host.numpy()
+        flat[2 * n : 3 * n] = src
+        flat[3 * n :] = old
+        with torch.cuda.stream(self._load_stream):
+            # the host allocator keeps the block until the copy has run
+            dev = torch.empty(host.shape, dtype=torch.int32, device=self.device)
+            dev.copy_(host, non_blocking=True)
+            self._tables_event = torch.cuda.Event()
+            self._tables_event.record(self._load_stream)
+        self._slots = dev[: 2 * n].view(torch.long)
+        self._src_map = dev[2 * n : 3 * n]
+        self._old_pos = dev[3 * n :] if hits else None
+
+    def _serve_slots(self, stream: torch.cuda.Stream, waited: bool = False) -> None:
+        """Orders ``stream``'s reads of the slots after their upload (``waited``:
+        it has waited for a later event of the Load stream)."""
+        if self._tables_event is None or stream.cuda_stream in self._slots_ready:
+            return
+        if not waited:
+            stream.wait_event(self._tables_event)
+        self._slots.record_stream(stream)
+        self._slots_ready.add(stream.cuda_stream)
 
     def _desc(self, layer_id: int) -> _native.KVDesc:
         desc = self._descs.get(layer_id)
@@ -468,6 +507,7 @@ class PagedBlendLoader:
             # the buffer was allocated on the Load stream; keep its memory
             # until the consuming stream is done with it
             self._buffers[layer_id].record_stream(current)
+            self._serve_slots(current, waited=True)
         if self.tracer is not None and self.tracer.enabled:
             self.tracer.emit(
                 "layer_prefetch_wait_enqueued",
@@ -489,6 +529,7 @@ class PagedBlendLoader:
             raise ValueError(
                 f"commit expects [2, {end}, {', '.join(map(str, self.row_shape))}] {self.dtype}"
             )
+        self._serve_slots(torch.cuda.current_stream(self.device))
         src = contiguous if contiguous[0].is_contiguous() and contiguous[1].is_contiguous() else contiguous.contiguous()
         es = src.element_size()
         rc = _native.load().cbk_paged_scatter(
