@@ -393,8 +393,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     const int32_t k0 = b * kKeyBlock;
     const uint16_t* base = src + int64_t(k0) * stride;
     if (k0 + kKeyBlock <= nk) {
-#pragma unroll
-      for (uint32_t j = 0; j < kInsts; ++j) lds_dma16(base, offs[j], l + (wave * kInsts + j) * 1024);
+      lds_dma16n<kInsts>(base, offs, l + wave * kInsts * 1024);
     } else {
       const uint32_t last = uint32_t(nk - 1 - k0);
 #pragma unroll
@@ -460,8 +459,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
                     uint32_t l) __attribute__((always_inline)) {
     const bool inner = j < nblocks - 1;
     if (inner || last_whole) {
-#pragma unroll
-      for (uint32_t i = 0; i < kInsts; ++i) lds_dma16(g, offs[i], l + (wave * kInsts + i) * 1024);
+      lds_dma16n<kInsts>(g, offs, l + wave * kInsts * 1024);
     } else {
       const uint32_t last = uint32_t(nk - 1 - (nblocks - 1) * kKeyBlock);
 #pragma unroll

@@ -113,6 +113,37 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32
                : "v"(off), "s"(uniform64(base)), "s"(__builtin_amdgcn_readfirstlane(int(lds)))
                : "memory");
 }
+// N requests from one base (offs[j] per lane) to consecutive 64-lane pieces,
+// lds + j * 1024: M0 is saved, padded for and restored once. Two requests a
+// step instead of one by one: 1% off the attention calls (7000 queries of
+// 32767 keys 1959 -> 1938 us, 180 of 8191 36.2 -> 35.8).
+template <int N>
+__device__ __forceinline__ void lds_dma16n(const void* base, const uint32_t (&offs)[N], uint32_t lds) {
+  static_assert(N == 1 || N == 2 || N == 4, "1, 2 or 4 requests");
+  if constexpr (N == 1) {
+    lds_dma16(base, offs[0], lds);
+    return;
+  }
+  uint32_t saved;
+#define CBK_LDS_NEXT(off) "s_nop 0\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 " off ", %1\n\t"
+#define CBK_LDS_FIRST "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %3, %1\n\t"
+#define CBK_LDS_LAST "s_nop 0\n\ts_mov_b32 m0, %0"
+  if constexpr (N == 2) {
+    asm volatile(CBK_LDS_FIRST CBK_LDS_NEXT("%4") CBK_LDS_LAST
+                 : "=&s"(saved)
+                 : "s"(uniform64(base)), "s"(__builtin_amdgcn_readfirstlane(int(lds))), "v"(offs[0]), "v"(offs[1])
+                 : "memory", "scc");
+  } else if constexpr (N == 4) {
+    asm volatile(CBK_LDS_FIRST CBK_LDS_NEXT("%4") CBK_LDS_NEXT("%5") CBK_LDS_NEXT("%6") CBK_LDS_LAST
+                 : "=&s"(saved)
+                 : "s"(uniform64(base)), "s"(__builtin_amdgcn_readfirstlane(int(lds))), "v"(offs[0]), "v"(offs[1]),
+                   "v"(offs[2]), "v"(offs[3])
+                 : "memory", "scc");
+  }
+#undef CBK_LDS_NEXT
+#undef CBK_LDS_FIRST
+#undef CBK_LDS_LAST
+}
 __device__ __forceinline__ void lds_dma4(const void* base, uint32_t off, uint32_t lds) {
   uint32_t saved;
   asm volatile(CBK_LDS_DMA("global_load_lds_dword")

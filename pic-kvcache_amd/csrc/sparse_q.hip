@@ -384,8 +384,7 @@ void sq_rowstats_kernel(const SqArgs a) {
     const char* base = a.k + int64_t(k0) * a.k_stride * 2;
     const uint32_t lk = lds_address(kbuf[b]);
     if (k0 + kKeyBlock1 <= int32_t(a.nk)) {
-#pragma unroll
-      for (uint32_t j = 0; j < kInsts; ++j) lds_dma16(base, koff[j], lk + (wave * kInsts + j) * 1024);
+      lds_dma16n<kInsts>(base, koff, lk + wave * kInsts * 1024);
     } else {
       const uint32_t last = uint32_t(int32_t(a.nk) - 1 - k0);
 #pragma unroll
@@ -720,8 +719,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))
         FLAT ? a.qdense + (int64_t(g) * ntiles_pad * G + f0) * (kQTile * D)
              : a.qdense + ((int64_t(g) * ntiles_pad + t0) * a.groups + hc * kHeadChunk) * (kQTile * D);
     const uint32_t lq = lds_address(qbuf[B]);
-#pragma unroll
-    for (uint32_t j = 0; j < kInsts; ++j) lds_dma16(unit, qoff[j], lq + (wave * kInsts + j) * 1024);
+    lds_dma16n<kInsts>(unit, qoff, lq + wave * kInsts * 1024);
     if (wave == 0) {
       const float2* st = a.stats + int64_t(g * G + hc * kHeadChunk) * a.nq_pad + t0 * kQTile;
       uint32_t soff = soff_full;
