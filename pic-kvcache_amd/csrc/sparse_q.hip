@@ -1,4 +1,4 @@
-// Sparse-Q attention-mass scores for gfx950 .
+// Sparse-Q attention-mass scores for gfx950.
 //
 // full[k] = sum_{h, q : pos_q >= k} softmax_k( r(Q[q,h] . K[k, h/G]) * scale )
 // where r rounds the dot product to the input dtype (the reference's bf16
@@ -14,7 +14,7 @@
 //             first-block maximum (online max / sum where that does not
 //             apply) in the log2 domain, merged across the 16 lanes that
 //             share a row -> (m, l) per (range, head, query)
-//   merge     the ranges' (m, l) of each row, in range order -> m + log2(l)
+//   merge     the ranges' (m, l) of each row, in a fixed order -> m + log2(l)
 //   colsum    one workgroup per (256-key block, query-unit range, kv head):
 //             each wave keeps its 64 keys' K fragments in registers and
 //             streams the range's query tiles (all G heads staged in LDS),
