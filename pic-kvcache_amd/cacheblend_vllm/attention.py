@@ -58,7 +58,12 @@ def blend_attention(
     # call: a captured graph then owns its own
     dtype_code = _native.DTYPE_CODES[query.dtype]
     nbytes = lib.cbk_blend_attention_workspace_bytes(nq, nk, hq, hkv, d, dtype_code)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
+    ws = None
+    if nbytes:
+        try:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device)
+        except torch.cuda.OutOfMemoryError:
+            nbytes = 0  # one range, which needs no scratch
     rc = lib.cbk_blend_attention_ws(
         query.data_ptr(), query.stride(0), pos.data_ptr(), nq,
         key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0), nk, hq, hkv, d,

@@ -143,3 +143,22 @@ def test_ranges_agree_with_one_range_far_above_the_first_blocks_maximum():
     assert torch.isfinite(got).all()
     # each side rounds probabilities and outputs once: 2 * 2 * 2^-8 of values up to 4.5
     assert float(diff.max()) <= 4 * 2.0 ** -8 * 4.5
+
+
+def test_no_memory_for_the_ranges(monkeypatch):
+    # the call needs no scratch without them
+    nq, nk, hq, hkv, d = 40, 3000, 8, 2, 128
+    q, k, v, pos = _inputs(nq, nk, hq, hkv, d, torch.bfloat16, seed=8)
+    q, k, v, pos = (t.to(DEV) for t in (q, k, v, pos))
+    want = blend_attention(q, k, v, pos, d ** -0.5)
+    empty = torch.empty
+
+    def full(*args, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.cuda.OutOfMemoryError("out of memory")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    got = blend_attention(q, k, v, pos, d ** -0.5)
+    # probabilities rounded against another reference, and the output: 2^-8 each, of values up to 4.5
+    assert float((got.float() - want.float()).abs().max()) <= 4 * 2.0 ** -8 * 4.5
