@@ -233,7 +233,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_kernel(const AttnF32Args
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
 
-  // the wave's rows with a term that is not finite (bit = row): redone below
+  // the wave's rows with a term that is not finite (bit = row): redone below.
+  // Rows past the last one count as little as their lanes do: their zeros
+  // times a value that is not finite are NaN too, and nothing of theirs may be
+  // read or written.
   uint32_t bad = 0;
   {
     const uint64_t lb = __ballot(!finite_bits(l));
@@ -248,6 +251,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_kernel(const AttnF32Args
       for (int g = 0; g < 4; ++g)
         if ((ob >> (16 * g)) & 0xffffu) bad |= 1u << (4 * g + i);
     }
+    bad &= uint32_t(__ballot(valid)) & 0xffffu;  // lanes 0..15 hold rows 0..15
   }
   const uint64_t rows_all = uint64_t(a.nq) * a.hq;
   // lane group grp holds rows 4 grp + i, dims 64 c + 4 (lane % 16) + e

@@ -100,6 +100,46 @@ def test_f32_values_past_a_position_do_not_reach_its_row():
     assert np.all(np.isnan(got[pos.numpy() >= 300]))
 
 
+def _attend_in_guards(q, k, v, pos, scale, ranges):
+    """``blend_attention`` through the C entry, ``out`` and the ranges' scratch
+    inside larger buffers: (out, whether the memory around both is untouched)."""
+    lib, (nq, hq, d), (nk, hkv, _) = _native.load(), q.shape, k.shape
+    code, guard = _native.DTYPE_CODES[q.dtype], 1 << 16
+    nbytes = lib.cbk_blend_attention_workspace_bytes(nq, nk, hq, hkv, d, code) if ranges else 0
+    assert (nbytes > 0) == ranges
+    out_bytes = nq * hq * d * q.element_size()
+    bufs = [torch.full((2 * guard + n,), 0x5A, dtype=torch.uint8, device=DEV) for n in (out_bytes, nbytes)]
+    out = bufs[0][guard:guard + out_bytes].view(q.dtype).view(nq, hq, d)
+    rc = lib.cbk_blend_attention_ws(
+        q.data_ptr(), hq * d, pos.data_ptr(), nq, k.data_ptr(), hkv * d, v.data_ptr(), hkv * d, nk, hq, hkv, d,
+        scale, code, out.data_ptr(), hq * d, bufs[1].data_ptr() + guard if ranges else None, nbytes,
+        _native.stream_handle(DEV))
+    _native.check(rc, "blend_attention")
+    whole = all(bool((b[:guard] == 0x5A).all()) and bool((b[-guard:] == 0x5A).all()) for b in bufs)
+    return out.cpu(), whole
+
+
+# a last row tile with and without rows past the end, the bad key in the
+# first, a middle and the last range of the last tile, and past the positions of the first
+@pytest.mark.parametrize("ranges", [False, True])
+@pytest.mark.parametrize("bad_key", [20, 500, 890])
+@pytest.mark.parametrize("nq,d", [(36, 64), (36, 66), (37, 128), (40, 64), (5, 100)])
+def test_f32_keys_that_are_not_finite_reach_the_rows_that_see_them_only(nq, d, bad_key, ranges):
+    nk, hq, hkv, scale = 900, 4, 2, 0.125
+    q, k, v, _ = _inputs(nq, nk, hq, hkv, d, seed=nq)
+    pos = torch.linspace(-1, nk - 1, nq).long()
+    want, mass, size = _f64(q, k, v, pos.clamp(min=0), scale)
+    k[bad_key, 0], v[bad_key, 1] = float("nan"), float("inf")
+    print(f"nq={nq} d={d} bad={bad_key} ranges={ranges}", flush=True)
+    got, whole = _attend_in_guards(*(t.to(DEV) for t in (q, k, v, pos)), scale, ranges)
+    assert whole
+    got, sees = got.numpy(), pos.numpy() >= bad_key
+    clean = ~sees & (pos.numpy() >= 0)
+    assert np.all(np.abs(got - want)[clean] <= _f32_bound(mass, size, d, nk, scale)[clean])
+    assert np.all(got[pos.numpy() < 0] == 0)
+    assert np.all(np.isnan(got[sees, :2])) and np.all(np.isposinf(got[sees, 2:]))
+
+
 # 16-bit rows around the 128-row tile, keys around the 32-key block and the
 # four-block rings, ranges in which rows see nothing, and both merge widths;
 # keys and queries in {-1, 0, 1} / 8, whose dot products are exact
