@@ -19,7 +19,8 @@ Per layer, on the Load stream (a default-priority side stream):
      scattered over the slab, in place -- the assembly kernel reads them
      from pinned host memory through a per-layer address table;
   2. ``cbk_blend_assemble`` (``_chunks`` for in-place reads) writes the
-     layer buffer in one pass: APC prefix from the pages, zeros for gaps,
+     layer buffer in one pass: APC prefix from the pages (as written by the
+     work the serving stream held when the loader was made), zeros for gaps,
      hit rows with their K RoPE-relocated from source to target positions;
   3. an event, waited on by ``get``.
 Two buffers alternate by layer parity; ``commit`` records a reuse event so
@@ -186,6 +187,13 @@ class PagedBlendLoader:
         self._tables_event: torch.cuda.Event | None = None
         self._slots_ready: set[int] = set()
         self._upload_tables(src, old, slots)
+        if self._load_stream is not None:
+            # the assemblies read what the serving stream has queued so far:
+            # the prefix's pages, the RoPE cache, slots converted on the
+            # device. The hits' DMA, on the copy stream, runs ahead of it.
+            queued = torch.cuda.Event()
+            queued.record(torch.cuda.current_stream(self.device))
+            self._load_stream.wait_event(queued)
         self._buffers: dict[int, torch.Tensor] = {}
         self._events: dict[int, torch.cuda.Event] = {}
         self._reuse_events: dict[int, torch.cuda.Event] = {}
