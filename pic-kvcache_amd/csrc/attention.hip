@@ -636,8 +636,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   // Fixed reference: after block 0 every row keeps the reference its first
   // step set (a logit of the row, so p <= 2^(max - m)) -- no per-logit
   // maximum, no threshold ballot. A row whose terms outgrew it (its sum past
-  // 2^100: a logit more than ~69 above the first block's maximum) or whose
-  // output is not finite is recomputed, workgroup-wide, with the lazy
+  // 2^100: a logit more than ~69 above the first block's maximum), whose
+  // output is not finite, or that was left without a reference although it
+  // sees keys (every logit of its first block -inf, which an f16 dot product
+  // below -65504 rounds to) is recomputed, workgroup-wide, with the lazy
   // rescaling.
   __shared__ uint32_t s_redo;
   if (nblocks > 0) {
@@ -645,6 +647,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     bool bad = false;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
+      bad |= m[t] == kNegInf && rpos[t] >= 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         bad |= !(ol[t][i] < 0x1p100f);

@@ -185,6 +185,46 @@ def test_ranges_agree_with_one_range_far_above_the_first_blocks_maximum():
     assert float(diff.max()) <= 4 * 2.0 ** -8 * 4.5
 
 
+@pytest.mark.parametrize("ranges", [False, True])
+@pytest.mark.parametrize("where", ["first block", "before low logits", "one range", "every range", "all"])
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 128), (torch.float16, 64), (torch.bfloat16, 128)])
+def test_16_bit_first_blocks_of_minus_infinity(dtype, d, where, ranges):
+    # rows whose logits in a range's first 32 keys are all -inf: in float16 a
+    # finite dot product below -65504 (heads of zeros beside them, in the same
+    # tiles), in bfloat16 a key of -inf
+    nq, nk, hq, hkv = 40, 4000, 4, 1
+    g = torch.Generator().manual_seed(6)
+    q = torch.ones(nq, hq, d)
+    k = torch.randint(-1, 2, (nk, hkv, d), generator=g) / 8
+    k[torch.arange(nk) % 100 == 99] = 0.0625  # some keys far above the others
+    if where == "before low logits":  # 2^-184 and less against a reference of 0
+        k[:], k[torch.arange(nk) % 100 == 99] = -2.0, -2.0 + 0.0625
+    value = -1024.0 if dtype == torch.float16 else -float("inf")
+    if dtype == torch.float16:
+        q[:, 1::2] = 0
+    splits = 31  # one per 128 keys
+    blocks = {"first block": [0], "before low logits": [0], "one range": [125 * 20 // splits], "all": range(125),
+              "every range": [125 * s // splits for s in range(splits)]}[where]
+    for b in blocks:
+        k[32 * b:32 * b + 32] = value
+    q, k, v = q.to(dtype), k.to(dtype), torch.randn(nk, hkv, d, generator=g).to(dtype)
+    pos = torch.arange(nk - nq, nk)
+    if ranges:
+        row = 8 + d * 4  # bytes of a partial row
+        assert _native.load().cbk_blend_attention_workspace_bytes(
+            nq, nk, hq, hkv, d, _native.DTYPE_CODES[dtype]) // (nq * hq * row) == splits
+    want, mass, _ = _f64(q, k.clamp(min=-1024.0), v, pos, 1.0)
+    if where == "all":  # no key has a weight: zero
+        rows = (q[..., 0] != 0).numpy()
+        want[rows], mass[rows] = 0, 0
+    print(f"{dtype} d={d} {where} ranges={ranges}", flush=True)
+    got, whole = _attend_in_guards(*(t.to(DEV) for t in (q, k, v, pos)), 1.0, ranges)
+    assert whole
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    close = np.abs(got.float().numpy() - want) <= 3 * u * mass + 1e-6
+    assert np.all(close)
+
+
 def test_no_memory_for_the_ranges(monkeypatch):
     # the call needs no scratch without them
     nq, nk, hq, hkv, d = 40, 3000, 8, 2, 128
