@@ -14,11 +14,11 @@
 //                   both 16-byte loads of 8 consecutive dims; the result
 //                   holds key 4*(lane/16)+i of row lane%16 in register i
 //   softmax         per row in the log2 domain against a fixed reference:
-//                   the maximum of the row's first block (a logit of the row,
-//                   so no term exceeds 2^(max - m)); no per-logit maximum in
-//                   the later blocks. A row whose sum outgrows it (2^100) is
-//                   recomputed with online maxima (lazily rescaled, the row's
-//                   32 keys of a block spread over its 4 lane groups)
+//                   the maximum of the context's first block (a logit of the
+//                   row, so no term exceeds 2^(max - m)); no per-logit maximum
+//                   in the other blocks. A row whose sum outgrows it (2^100)
+//                   is recomputed with online maxima (lazily rescaled, the
+//                   row's 32 keys of a block spread over its 4 lane groups)
 //   O += P . V      v_mfma_f32_16x16x32_{bf16,f16}: the two halves' S^T
 //                   registers, concatenated, are the A operand (row lane%16,
 //                   keys 4*(lane/16)..+3 and 16+4*(lane/16)..+3: the
@@ -594,12 +594,14 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     while (b < end) single(kind, fix, b);
   };
   // one pass over the blocks; the first step always takes the lazy path (it
-  // sets each row's reference from block 0, where every row with a position
-  // sees key 0 at least)
+  // sets the references that are not set yet from the range's first block)
   auto pass = [&](auto fix) __attribute__((always_inline)) {
     // the first kBuffers blocks of K and two fewer of V ahead of step 0, in
     // the order the steps wait for them; then every wave takes steps 0 ..
-    // nblocks (the requests and barriers of each)
+    // nblocks (the requests and barriers of each). A range past the first also
+    // reads the context's block 0, into the V buffer that step 1 fills first.
+    const bool context_ref = decltype(fix)::value && b_lo > 0;
+    if (context_ref) lds_dma16n<kInsts>(a.k, koff, lds_address(vbuf[kBuffers - 1]) + wave * kInsts * 1024);
     request(0, k_range, a.k_stride, koff, kbuf);
     request(1, k_range, a.k_stride, koff, kbuf);
 #pragma unroll
@@ -607,8 +609,24 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
       request(2 + j, k_range, a.k_stride, koff, kbuf);
       request(j, v_range, a.v_stride, voff, vbuf);
     }
-    CBK_WAIT_VM_LGKM0((2 * (kBuffers - 2) + 1) * kInsts);  // K(0) has landed
+    CBK_WAIT_VM_LGKM0((2 * (kBuffers - 2) + 1) * kInsts);  // K(0), and the context's block 0, have landed
     asm volatile("s_barrier" ::: "memory");
+    if (context_ref && b_w > 0) {
+      qk_block<F16, D, RT>((const uint16_t*)(__attribute__((address_space(3))) const uint16_t*)(size_t)lds_address(
+                               vbuf[kBuffers - 1]),
+                           off, qf, sa);
+      float lm[RT];
+      logits_block<F16, RT, true>(sa, -key0, a.scale, rpos, lm, grp);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        float bm = fmaxf(lm[t], __shfl_xor(lm[t], 16));
+        bm = fmaxf(bm, __shfl_xor(bm, 32));
+        const float mn = bm * kLog2e + 1.f;
+        m[t] = mn;
+        nms[t] = mn == kNegInf ? 0.f : -mn;
+        thr[t] = mn == kNegInf ? kNegInf : -kNegInf;  // the first step keeps it
+      }
+    }
     if (b_w > 0) {
       qk_block<F16, D, RT>((const uint16_t*)(__attribute__((address_space(3))) const uint16_t*)(size_t)lds_address(
                                kbuf[0]),
@@ -633,9 +651,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
     for (; b <= nblocks; ++b) step(none(), no(), any(), fix, b, sa, sb, pa, pb);
     CBK_WAIT_VM_LGKM0(0);  // no LDS write in flight past this point
   };
-  // Fixed reference: after block 0 every row keeps the reference its first
-  // step set (a logit of the row, so p <= 2^(max - m)) -- no per-logit
-  // maximum, no threshold ballot. A row whose terms outgrew it (its sum past
+  // Fixed reference: every row keeps the maximum of the context's block 0,
+  // where a row with a position sees key 0 at least (a logit of the row, so
+  // p <= 2^(max - m)) -- no per-logit maximum, no threshold ballot. The ranges
+  // share it: the probabilities are rounded as one range rounds them, and the
+  // first keys, whose logits tend to be a prompt's largest, serve all of them
+  // (a float16 probability overflows 11 above the reference; with each range's
+  // own first block 3000 queries of 16000 keys, logits of deviation 4 under a
+  // first key above them all, took 416 us with the second passes, 332 without
+  // ranges, and take 239). A row whose terms outgrew it (its sum past
   // 2^100: a logit more than ~69 above the first block's maximum), whose
   // output is not finite, or that was left without a reference although it
   // sees keys (every logit of its first block -inf, which an f16 dot product
