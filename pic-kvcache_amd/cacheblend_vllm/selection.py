@@ -333,7 +333,7 @@ def sparse_q_rows(gap_mask: torch.Tensor, tail_query_tokens: int, radius: int):
     # the counts behind the rows: one allocation
     rows = torch.empty(n + lib.cbk_sparse_q_rows_counts(n), dtype=torch.long, device=dev)
     counts = rows[n:]
-    rc = lib.cbk_sparse_q_rows(gap.data_ptr(), n, tail_query_tokens, radius, forced.data_ptr(), rows.data_ptr(),
+    rc = lib.cbk_sparse_q_rows(gap.data_ptr(), n, int(tail_query_tokens), int(radius), forced.data_ptr(), rows.data_ptr(),
                                counts.data_ptr(), _native.stream_handle(dev))
     _native.check(rc, "sparse_q_rows")
     gap_count = int(counts[0].item())

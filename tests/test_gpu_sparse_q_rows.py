@@ -1,10 +1,12 @@
 """The Sparse-Q queries and forced tokens of a gap mask: one call against the
 mask functions on torch, for every form of mask and tail."""
 
+import numpy as np
 import pytest
 import torch
 
 from cacheblend_vllm import selection as S
+from cacheblend_vllm.config import CacheBlendConfig
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
@@ -33,3 +35,16 @@ def test_rows_match_the_mask_functions(n, radius):
             assert got_count == count
             assert torch.equal(rows, want)
             assert torch.equal(got, forced)
+
+
+@pytest.mark.parametrize("block", [16, np.int64(16), 16.0])
+@pytest.mark.parametrize("tail", [64, np.int64(64)])
+def test_sizes_of_any_whole_number_type(block, tail):
+    n, g = 300, torch.Generator().manual_seed(5)
+    q, k = torch.randn(n, 2, 64, generator=g).to(DEV), torch.randn(n, 1, 64, generator=g).to(DEV)
+    index = torch.arange(n, device=DEV)
+    config = CacheBlendConfig.from_extra_config({"selection_strategy": "sparse_q", "tail_query_tokens": tail})
+    for gap in (torch.zeros(n, dtype=torch.bool), torch.arange(n) == 100):
+        want_q, want, _ = S.sparse_q_masks(gap.to(DEV), 64, 16)
+        _, forced, stats = S.BlendSelector(config, block)._sparse_q_scores(q, k, index, gap.to(DEV), 0.125)
+        assert torch.equal(forced, want) and stats["sparse_query_tokens"] == int(want_q.sum())
