@@ -24,7 +24,8 @@
 //
 // Rows with a term that is not finite are computed again one by one, over
 // their visible keys only: the blocks multiply a masked key's probability of
-// zero with its value row, which may hold anything.
+// zero with its value row, which may hold anything. So are rows without a
+// sum, in natural units: logits past 1 / log2 e of the type's range.
 #include <cmath>
 
 #include "attention_split.hpp"
@@ -233,13 +234,14 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_kernel(const AttnF32Args
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
 
-  // the wave's rows with a term that is not finite (bit = row): redone below.
+  // the wave's rows with a term that is not finite, or with keys but no sum
+  // (logits that are finite by themselves, -inf times log2 e): redone below.
   // Rows past the last one count as little as their lanes do: their zeros
   // times a value that is not finite are NaN too, and nothing of theirs may be
   // read or written.
   uint32_t bad = 0;
   {
-    const uint64_t lb = __ballot(!finite_bits(l));
+    const uint64_t lb = __ballot(!finite_bits(l) || (l == 0.f && b_lo < b_hi && rpos >= b_lo * kKeys));
     bad = uint32_t((lb | (lb >> 16) | (lb >> 32) | (lb >> 48)) & 0xffffu);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_kernel(const AttnF32Args
       const uint64_t id = split * rows_all + uint64_t(oq) * a.hq + oh;
       dst = a.parts.o + id * a.d;
       f = 1.f;
-      if (row == 0) a.parts.ml[id] = make_float2(rm, rl);
+      if (row == 0) a.parts.ml[id] = make_float2(0.5f * rm, rl);
     }
 #pragma unroll
     for (int c = 0; c < CC; ++c) {
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_kernel(const AttnF32Args
     } else {
       const uint64_t id = split * rows_all + uint64_t(oq) * a.hq + oh;
       dst = a.parts.o + id * a.d;
-      if (lane == 0) a.parts.ml[id] = make_float2(fm * kLog2e, fl);
+      if (lane == 0) a.parts.ml[id] = make_float2(fm * (0.5f * kLog2e), fl);
     }
     if (lane < a.d) dst[lane] = o0 * f;
     if (lane + 64 < a.d) dst[lane + 64] = o1 * f;

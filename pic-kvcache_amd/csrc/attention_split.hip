@@ -30,6 +30,7 @@ __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(const AttnPar
                                                                    uint32_t d, const int64_t* pos, T* out,
                                                                    int64_t out_stride, bool nan_empty) {
   constexpr int E = N ? N : 4;  // d <= 128
+  constexpr bool F32 = sizeof(T) == 4;
   typedef float VecN __attribute__((ext_vector_type(E)));
   const uint32_t lane = threadIdx.x & 31;
   const uint64_t rows = uint64_t(nq) * hq;
@@ -41,7 +42,7 @@ __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(const AttnPar
 #pragma unroll
   for (int off = 16; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 32));
   // a range without visible keys for the row: its sum is 0, its output may be unwritten
-  const float w = ml.y == 0.f ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+  const float w = ml.y == 0.f ? 0.f : __builtin_amdgcn_exp2f((F32 ? 2.f : 1.f) * (ml.x - m));
   float l = ml.y == 0.f ? 0.f : w * ml.y;
 #pragma unroll
   for (int off = 16; off >= 1; off >>= 1) l += __shfl_xor(l, off, 32);

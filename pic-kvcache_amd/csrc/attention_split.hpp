@@ -11,8 +11,9 @@ namespace cbk {
 constexpr int kAttnKeyBlock = 32;  // keys per block of the attention kernels
 
 // Partial results of `splits` key ranges: for range s and row r = query *
-// hq + head, ml[s * rows + r] = (maximum in log2 units, sum of 2^(x - maximum))
-// and o[(s * rows + r) * d ..] the sum of 2^(x - maximum) * value, float32.
+// hq + head, ml[s * rows + r] = (reference m in log2 units, sum of 2^(x - m))
+// and o[(s * rows + r) * d ..] the sum of 2^(x - m) * value, float32. From
+// float32 inputs m is halved: it holds every logit of the type that way.
 struct AttnParts {
   uint32_t splits;  // 1: no partials, the workgroups write the output
   float2* ml;

@@ -140,6 +140,24 @@ def test_f32_keys_that_are_not_finite_reach_the_rows_that_see_them_only(nq, d, b
     assert np.all(np.isnan(got[sees, :2])) and np.all(np.isposinf(got[sees, 2:]))
 
 
+# logits around the type's lowest and largest value, which times log2 e are
+# infinite
+@pytest.mark.parametrize("ranges", [False, True])
+@pytest.mark.parametrize("logits", [(-3e38, -3e38), (3e38, 3e38), (-3e38, -2.5e38), (-3e38, 1.0), (-1.5e38, -2.9e38)])
+def test_f32_logits_of_any_size(logits, ranges):
+    nq, nk, hq, hkv, d = 20, 900, 2, 1, 64
+    q, k, v, _ = _inputs(nq, nk, hq, hkv, d, seed=5)
+    q.zero_(), k.zero_()
+    q[..., 0], k[..., 0] = 1.0, logits[0]
+    k[torch.arange(nk) % 3 == 1, :, 0] = logits[1]
+    k[600:, :, 0] = max(logits)  # the last ranges hold one value alone
+    pos = torch.arange(nq) * 45 + 44
+    want, mass, size = _f64(q, k, v, pos, 1.0)
+    got, whole = _attend_in_guards(*(t.to(DEV) for t in (q, k, v, pos)), 1.0, ranges)
+    assert whole
+    assert np.all(np.abs(got.numpy() - want) <= _f32_bound(mass, 0.0, d, nk, 1.0))
+
+
 # 16-bit rows around the 128-row tile, keys around the 32-key block and the
 # four-block rings, ranges in which rows see nothing, and both merge widths;
 # keys and queries in {-1, 0, 1} / 8, whose dot products are exact
