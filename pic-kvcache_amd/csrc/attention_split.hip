@@ -41,8 +41,13 @@ __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(const AttnPar
   float m = ml.x;
 #pragma unroll
   for (int off = 16; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 32));
-  // a range without visible keys for the row: its sum is 0, its output may be unwritten
+  // a range without visible keys for the row: its sum is 0, its output may be
+  // unwritten (never in float32)
   const float w = ml.y == 0.f ? 0.f : __builtin_amdgcn_exp2f((F32 ? 2.f : 1.f) * (ml.x - m));
+  // every other output counts, also with a weight of 0 (an infinity in it is
+  // NaN then, as in one range)
+  const uint64_t any = __ballot(F32 || ml.y != 0.f);
+  const uint32_t use = uint32_t((threadIdx.x & 32) ? any >> 32 : any);
   float l = ml.y == 0.f ? 0.f : w * ml.y;
 #pragma unroll
   for (int off = 16; off >= 1; off >>= 1) l += __shfl_xor(l, off, 32);
@@ -53,7 +58,7 @@ __global__ __launch_bounds__(kMergeThreads) void attn_merge_kernel(const AttnPar
 #pragma unroll 8
   for (uint32_t s = 0; s < S; ++s) {
     const float ws = __shfl(w, int(s), 32);
-    const bool used = ws != 0.f;
+    const bool used = (use >> s) & 1u;
     if constexpr (N != 0) {
       const VecN v = used ? *reinterpret_cast<const VecN*>(o + s * rows * d + lane * N) : VecN(0.f);
 #pragma unroll

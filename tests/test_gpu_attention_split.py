@@ -141,7 +141,7 @@ def test_f32_keys_that_are_not_finite_reach_the_rows_that_see_them_only(nq, d, b
 
 
 # logits around the type's lowest and largest value, which times log2 e are
-# infinite
+# infinite, and an infinite value whose key's probability is 0
 @pytest.mark.parametrize("ranges", [False, True])
 @pytest.mark.parametrize("logits", [(-3e38, -3e38), (3e38, 3e38), (-3e38, -2.5e38), (-3e38, 1.0), (-1.5e38, -2.9e38)])
 def test_f32_logits_of_any_size(logits, ranges):
@@ -156,6 +156,12 @@ def test_f32_logits_of_any_size(logits, ranges):
     got, whole = _attend_in_guards(*(t.to(DEV) for t in (q, k, v, pos)), 1.0, ranges)
     assert whole
     assert np.all(np.abs(got.numpy() - want) <= _f32_bound(mass, 0.0, d, nk, 1.0))
+    if logits == (-3e38, 1.0):
+        # seen by all rows, at a probability of 0 of those that see a key past the first ranges
+        k[:128, :, 0], v[0, 0, 3] = logits[0], float("inf")
+        got, _ = _attend_in_guards(*(t.to(DEV) for t in (q, k, v, pos)), 1.0, ranges)
+        assert bool(torch.isnan(got[3:, :, 3]).all()) and not bool(torch.isfinite(got[..., 3]).any())
+        assert bool(torch.isfinite(got[..., 4:]).all())
 
 
 # 16-bit rows around the 128-row tile, keys around the 32-key block and the
