@@ -63,8 +63,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kWaves = 4;
 constexpr int kRowTiles = 2;  // 16-row tiles per wave
 constexpr int kKeyBlock = kAttnKeyBlock;
-// Workgroups per CU that the key ranges aim at: as many as are resident.
-constexpr uint32_t per_cu(int64_t head_dim) { return head_dim == 64 ? 3 : 2; }
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kNegInf = -__builtin_inff();
@@ -761,12 +759,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
 namespace cbk {
 namespace {
 
-// Key ranges of a launch (attn_splits) for inputs that passed the checks.
+// Key ranges of a launch for inputs that passed the checks.
 uint32_t launch_splits(int64_t nq, int64_t nk, int64_t hq, int64_t hkv, int64_t head_dim, int32_t dtype) {
   const uint64_t nrows = uint64_t(nq) * uint64_t(hq / hkv);
   const uint64_t rows_per_wg = dtype == CBK_DTYPE_F32 ? kAttnF32Rows : 16 * kRowTiles * kWaves;
   const uint64_t groups = (nrows + rows_per_wg - 1) / rows_per_wg * uint64_t(hkv);
-  return attn_splits(groups, dtype == CBK_DTYPE_F32 ? kAttnF32PerCu : per_cu(head_dim), nk);
+  if (dtype == CBK_DTYPE_F32) return attn_f32_splits(groups, nk);
+  return attn_splits(groups, uint64_t(nq) * uint64_t(hq), nk, head_dim);
 }
 
 int check_sizes(int64_t nq, int64_t nk, int64_t hq, int64_t hkv) {

@@ -3,16 +3,17 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "attention_split.hpp"
 
 namespace cbk {
 namespace {
 
-// A range holds at least 4 of the kernels' 32-key blocks of the longest row:
-// shorter ones cost more in partials than they save.
 constexpr uint32_t kMaxSplits = 32;
-constexpr int64_t kMinKeysPerSplit = 128;
+constexpr uint32_t kMinBlocksPerSplit = 3;
+// float32: shorter ranges cost more in partials than they save
+constexpr int64_t kMinKeysPerSplitF32 = 128;
 constexpr int kMergeThreads = 256;
 
 template <typename T> __device__ __forceinline__ T to_out(float v);
@@ -104,15 +105,38 @@ int launch_merge_t(const AttnParts& parts, uint32_t nq, uint32_t hq, uint32_t d,
 
 }  // namespace
 
-uint32_t attn_splits(uint64_t groups, uint32_t per_cu, int64_t nk) {
+uint32_t attn_splits(uint64_t groups, uint64_t rows, int64_t nk, int64_t d) {
   int cus = 0;
   if (groups == 0 || device_cus(&cus)) return 1;
-  const uint64_t want = uint64_t(per_cu) * uint32_t(cus);
+  struct Cost { double start, step, share, merge, range, rate; };
+  const Cost c = d == 64 ? Cost{6.5, 0.48, 0.146, 3.1, 0.21, 4.3e6} : Cost{8.1, 0.59, 0.25, 2.5, 0.16, 5.1e6};
+  const double blocks = double((nk + kAttnKeyBlock - 1) / kAttnKeyBlock);
+  const double busy = double(groups) * blocks * c.share / cus;
+  auto cost = [&](uint32_t s) {
+    const double chain = c.start + blocks / s * c.step;
+    const double pass = std::sqrt(std::sqrt(chain * chain * chain * chain + busy * busy * busy * busy));
+    return s == 1 ? pass : pass + c.merge + s * (c.range + double(rows) * double(d + 2) * 8 / c.rate);
+  };
+  uint32_t best = 1;
+  double least = 0.97 * cost(1);  // no partials for less than 3%
+  const uint32_t most = uint32_t(std::min<double>(kMaxSplits, blocks / kMinBlocksPerSplit));
+  for (uint32_t s = 2; s <= most; ++s)
+    if (const double t = cost(s); t < least) {
+      least = t;
+      best = s;
+    }
+  return best;
+}
+
+uint32_t attn_f32_splits(uint64_t groups, int64_t nk) {
+  int cus = 0;
+  if (groups == 0 || device_cus(&cus)) return 1;
+  const uint64_t want = uint64_t(kAttnF32PerCu) * uint32_t(cus);
   // one round of workgroups where that takes three or more ranges; with fewer
   // the ranges are long, and two shorter rounds even out the tiles' lengths
   uint64_t s = want / groups;
   if (s < 3) s = 2 * want / groups;
-  s = std::min<uint64_t>(s, uint64_t(nk / kMinKeysPerSplit));
+  s = std::min<uint64_t>(s, uint64_t(nk / kMinKeysPerSplitF32));
   return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(s, kMaxSplits)));
 }
 

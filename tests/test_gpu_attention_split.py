@@ -226,17 +226,15 @@ def test_16_bit_first_blocks_of_minus_infinity(dtype, d, where, ranges):
     value = -1024.0 if dtype == torch.float16 else -float("inf")
     if dtype == torch.float16:
         q[:, 1::2] = 0
-    splits = 31  # one per 128 keys
+    splits = _native.load().cbk_blend_attention_workspace_bytes(
+        nq, nk, hq, hkv, d, _native.DTYPE_CODES[dtype]) // (nq * hq * (8 + 4 * d))
+    assert splits > 8
     blocks = {"first block": [0], "before low logits": [0], "one range": [125 * 20 // splits], "all": range(125),
               "every range": [125 * s // splits for s in range(splits)]}[where]
     for b in blocks:
         k[32 * b:32 * b + 32] = value
     q, k, v = q.to(dtype), k.to(dtype), torch.randn(nk, hkv, d, generator=g).to(dtype)
     pos = torch.arange(nk - nq, nk)
-    if ranges:
-        row = 8 + d * 4  # bytes of a partial row
-        assert _native.load().cbk_blend_attention_workspace_bytes(
-            nq, nk, hq, hkv, d, _native.DTYPE_CODES[dtype]) // (nq * hq * row) == splits
     want, mass, _ = _f64(q, k.clamp(min=-1024.0), v, pos, 1.0)
     if where == "all":  # no key has a weight: zero
         rows = (q[..., 0] != 0).numpy()
@@ -267,6 +265,19 @@ def test_16_bit_ranges_round_the_probabilities_of_one_range(dtype, d, share):
     differ = float((a != b).float().mean())
     print(f"share of outputs that differ {differ:.5f}", flush=True)
     assert differ <= share
+
+
+# short contexts and full row tiles take one range (several were slower), long
+# contexts of few rows as many as fill the chip
+@pytest.mark.parametrize("nq,nk,hq,hkv,d,least,most", [
+    (64, 256, 32, 8, 128, 1, 1), (256, 256, 8, 2, 64, 1, 1), (900, 1000, 32, 8, 128, 1, 1),
+    (2000, 4000, 32, 8, 128, 1, 1), (7000, 32767, 32, 4, 128, 1, 1), (1000, 4000, 32, 8, 128, 2, 4),
+    (1, 32767, 8, 8, 128, 8, 32), (180, 8191, 32, 8, 64, 6, 16),
+])
+def test_16_bit_ranges_where_they_pay(nq, nk, hq, hkv, d, least, most):
+    code = _native.DTYPE_CODES[torch.bfloat16]
+    nbytes = _native.load().cbk_blend_attention_workspace_bytes(nq, nk, hq, hkv, d, code)
+    assert least <= max(1, nbytes // (nq * hq * (8 + 4 * d))) <= most
 
 
 def test_no_memory_for_the_ranges(monkeypatch):
