@@ -1293,7 +1293,7 @@ __device__ __forceinline__ void block_digit(const uint32_t* hist, uint32_t k, ui
 
 template <int NT, int ITEMS>
 __global__ __launch_bounds__(NT) void sel_block_kernel(const SelArgs a) {
-  extern __shared__ uint32_t window[];  // NT * ITEMS prefix counts of gaps, r > 0
+  extern __shared__ uint32_t window[];  // NT * ITEMS prefix counts of gaps (r > 0), then the selected tokens
   __shared__ __attribute__((aligned(16))) uint32_t hist[4096];
   __shared__ uint32_t scan[NT / 64], scan2[NT / 64], digit[2];
   const uint32_t i0 = threadIdx.x * ITEMS;
@@ -1414,9 +1414,14 @@ __global__ __launch_bounds__(NT) void sel_block_kernel(const SelArgs a) {
   uint32_t total;
   uint32_t pos = block_exclusive_scan<NT>(__popc(write), scan2, &total);
   if (threadIdx.x == 0) *a.out_count = int64_t(total);
+  // through LDS (a word of padding per ITEMS), so that a wave's stores are
+  // consecutive: 15.5 -> 10.3 us for 16384 tokens all selected
+  auto slot = [](uint32_t p) { return p + p / ITEMS; };
 #pragma unroll
   for (int e = 0; e < ITEMS; ++e)
-    if (write >> e & 1u) a.out_idx[pos++] = int64_t(i0 + e);
+    if (write >> e & 1u) window[slot(pos++)] = i0 + e;
+  __syncthreads();
+  for (uint32_t j = threadIdx.x; j < total; j += NT) a.out_idx[j] = int64_t(window[slot(j)]);
 }
 
 __global__ void write_zero_count_kernel(int64_t* out_count) { *out_count = 0; }
@@ -1500,23 +1505,24 @@ int launch_onepass(const SelArgs& a, int64_t n, int64_t radius, hipStream_t stre
   return launch_status("select (one launch)");
 }
 
-// Tokens that the one-block select takes, 8 or 16 a thread. us a select,
-// one-launch form before -> one block: 1537 tokens 15.5 -> 8.0, 8192 17.5 -> 8.4,
-// 16384 17.6 -> 13.0; with a dilation of 16 18.5 -> 9.1, 18.6 -> 10.3, 18.9 ->
-// 16.2 (past that one CU's LDS passes take longer than the grid's barriers).
+// Tokens that the one-block select takes, 8 or 16 a thread (past that one CU's
+// LDS passes take longer than the grid's barriers). us a select, one-launch
+// form -> one block, 5% of the tokens gaps: 1537 tokens 15.9 -> 8.2, 8192 16.2
+// -> 8.6, 16384 17.3 -> 12.4; dilated by 16, most tokens selected, 19.2 -> 9.5,
+// 19.0 -> 10.6, 19.2 -> 16.0 (20.4 with stores straight from the registers).
 constexpr int64_t kBlockTokens = 16384;
 
 template <int NT, int ITEMS>
-int launch_block_t(const SelArgs& a, int64_t radius, hipStream_t stream) {
-  const size_t lds = radius > 0 ? size_t(NT) * ITEMS * sizeof(uint32_t) : 0;
+int launch_block_t(const SelArgs& a, hipStream_t stream) {
+  const size_t lds = size_t(NT) * (ITEMS + 1) * sizeof(uint32_t);
   hipLaunchKernelGGL((sel_block_kernel<NT, ITEMS>), dim3(1), dim3(NT), lds, stream, a);
   return launch_status("select (one block)");
 }
 
-int launch_block_select(const SelArgs& a, int64_t n, int64_t radius, hipStream_t stream) {
-  if (n <= 2048) return launch_block_t<256, 8>(a, radius, stream);
-  if (n <= 8192) return launch_block_t<1024, 8>(a, radius, stream);
-  return launch_block_t<1024, 16>(a, radius, stream);
+int launch_block_select(const SelArgs& a, int64_t n, hipStream_t stream) {
+  if (n <= 2048) return launch_block_t<256, 8>(a, stream);
+  if (n <= 8192) return launch_block_t<1024, 8>(a, stream);
+  return launch_block_t<1024, 16>(a, stream);
 }
 
 // header_zeroed: an earlier launch on the stream cleared the kHeader counter
@@ -1559,7 +1565,7 @@ int launch_select(const float* scores, const uint8_t* gap, const uint8_t* forced
   a.bar_extra = give_up ? 1u : 0u;
   // one block's tokens: everything in its LDS (CBK_SELECT_TEST_GIVE_UP asks
   // for the grid barrier, CBK_SELECT_MULTI_LAUNCH for the launches below)
-  if (flags == 0 && n <= kBlockTokens) return launch_block_select(a, n, radius, stream);
+  if (flags == 0 && n <= kBlockTokens) return launch_block_select(a, n, stream);
   if (!header_zeroed) hipLaunchKernelGGL(sel_zero_kernel, dim3(1), dim3(kSelThreads), 0, stream, a.ws);
   // one launch when every tile's block can be resident at once
   if ((flags & CBK_SELECT_MULTI_LAUNCH) == 0) {
