@@ -272,7 +272,7 @@ def test_16_bit_ranges_round_the_probabilities_of_one_range(dtype, d, share):
 @pytest.mark.parametrize("nq,nk,hq,hkv,d,least,most", [
     (64, 256, 32, 8, 128, 1, 1), (256, 256, 8, 2, 64, 1, 1), (900, 1000, 32, 8, 128, 1, 1),
     (2000, 4000, 32, 8, 128, 1, 1), (7000, 32767, 32, 4, 128, 1, 1), (1000, 4000, 32, 8, 128, 2, 4),
-    (1, 32767, 8, 8, 128, 8, 32), (180, 8191, 32, 8, 64, 6, 16),
+    (1, 32767, 8, 8, 128, 8, 32), (180, 8191, 32, 8, 64, 6, 16), (1, 255, 1, 1, 64, 1, 1), (1, 255, 8, 8, 128, 1, 1),
 ])
 def test_16_bit_ranges_where_they_pay(nq, nk, hq, hkv, d, least, most):
     code = _native.DTYPE_CODES[torch.bfloat16]
