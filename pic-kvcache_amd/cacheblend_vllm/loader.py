@@ -250,7 +250,7 @@ class PagedBlendLoader:
             return
         n, hits = src.size, old.size
         host = torch.empty(2 * n + n + hits, dtype=torch.int32, pin_memory=True)
-        host[: 2 * n].view(torch.long).copy_(slots)
+        host[: 2 * n].view(torch.long).copy_(slots.reshape(-1)[:n])
         flat = host.numpy()
         flat[2 * n : 3 * n] = src
         flat[3 * n :] = old

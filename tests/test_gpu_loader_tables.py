@@ -20,7 +20,8 @@ DEV = torch.device("cuda", 0)
 
 @pytest.mark.parametrize("slots_on", ["cpu", "cuda"])
 @pytest.mark.parametrize("streams", [1, 3])
-def test_commits_wait_for_the_slots(slots_on, streams):
+@pytest.mark.parametrize("column", [False, True])  # a column of slots, or a flat list
+def test_commits_wait_for_the_slots(slots_on, streams, column):
     heads, dim, block, blocks, end, prefix = 2, 64, 16, 40, 333, 32
     g = torch.Generator().manual_seed(7)
     load = torch.cuda.Stream()
@@ -34,8 +35,8 @@ def test_commits_wait_for_the_slots(slots_on, streams):
     del junk
     with torch.cuda.stream(load):
         torch.cuda._sleep(20_000_000)
-    loader = PagedBlendLoader(layers, PinnedChunkStore(256, 1 << 20), "r", BlendPlan(prefix, end, 0, ()), slots,
-                              block, CacheBlendConfig.from_extra_config({}), load_stream=load)
+    loader = PagedBlendLoader(layers, PinnedChunkStore(256, 1 << 20), "r", BlendPlan(prefix, end, 0, ()),
+                              slots[:, None] if column else slots, block, CacheBlendConfig.from_extra_config({}), load_stream=load)
     for i, stream in enumerate(serving):
         with torch.cuda.stream(stream):
             loader.commit(i, rows[i])
