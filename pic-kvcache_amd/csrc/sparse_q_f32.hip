@@ -20,7 +20,8 @@
 // MFMA layout (checked on gfx950): A[i][k] in lane i + 16 k, B[k][j] in lane
 // j + 16 k, D[i][j] in lane j + 16 (i / 4), register i % 4.
 //
-// Head sizes above 128 take one lane per logit.
+// Head sizes above 128, and more keys than one launch of the column pass
+// holds, take one lane per logit.
 #include <algorithm>
 
 #include "sparse_q.hpp"
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(kThreads) void sq_cols_f32_kernel(const SqArgs a) {
   if (grp == 0 && key < a.nk) a.partial[(int64_t(split) * a.hkv + g) * a.nk + key] = acc;
 }
 
-// ------------------------------------------------ head sizes above 128
+// ------------------------------------------------ one lane per logit
 
 // rowstats: one wavefront per (query, head); lanes stride over keys.
 __global__ __launch_bounds__(kThreads) void sq_rowstats_f32_kernel(const SqArgs a) {
@@ -316,23 +317,24 @@ uint32_t ranges(uint64_t units, int cus, uint32_t most) {
 }  // namespace
 
 int launch_sq_f32(SqArgs& a, hipStream_t stream) {
-  if (a.d > 128) {
+  int cus = 0;
+  if (int rc = device_cus(&cus)) return rc;
+  const uint64_t rows = uint64_t(a.nq) * a.groups;
+  const uint64_t u1 = (rows + kTile - 1) / kTile * a.hkv, u2 = (uint64_t(a.nk) + kTile - 1) / kTile * a.hkv;
+  const uint32_t row_chunks = ranges(u1, cus, max_row_chunks(uint64_t(a.hq) * a.nq_pad));
+  const uint32_t col_splits = ranges(u2, cus, kMaxColSplits);
+  // a launch holds 2^32 threads: keys past 2^30 / hkv take a thread each
+  if (a.d > 128 || rows >= (uint64_t(1) << 31) || u1 * row_chunks * kThreads >= (uint64_t(1) << 32) ||
+      u2 * col_splits * kThreads >= (uint64_t(1) << 32)) {
     const uint64_t items = uint64_t(a.nq) * a.hq;
     hipLaunchKernelGGL(sq_rowstats_f32_kernel, dim3(uint32_t((items + 3) / 4)), dim3(kThreads), 0, stream, a);
     hipLaunchKernelGGL(sq_colsum_f32_kernel, dim3(uint32_t((uint64_t(a.nk) * a.hkv + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, stream, a);
     return CBK_OK;
   }
-  int cus = 0;
-  if (int rc = device_cus(&cus)) return rc;
-  const uint64_t rows = uint64_t(a.nq) * a.groups;
-  CBK_REQUIRE(rows < (uint64_t(1) << 31), "sparse_q: %llu rows per KV head exceed one launch", (unsigned long long)rows);
-  const uint64_t u1 = (rows + kTile - 1) / kTile * a.hkv, u2 = (uint64_t(a.nk) + kTile - 1) / kTile * a.hkv;
-  a.row_chunks = ranges(u1, cus, max_row_chunks(uint64_t(a.hq) * a.nq_pad));
-  a.col_splits = ranges(u2, cus, kMaxColSplits);
-  CBK_REQUIRE(u1 * a.row_chunks * kThreads < (uint64_t(1) << 32) && u2 * a.col_splits * kThreads < (uint64_t(1) << 32),
-              "sparse_q: %llu rows x %u keys exceed one launch", (unsigned long long)rows, a.nk);
-  const uint32_t g1 = uint32_t(u1 * a.row_chunks), g2 = uint32_t(u2 * a.col_splits);
+  a.row_chunks = row_chunks;
+  a.col_splits = col_splits;
+  const uint32_t g1 = uint32_t(u1 * row_chunks), g2 = uint32_t(u2 * col_splits);
   const int64_t align[5] = {a.q_stride * 4, a.k_stride * 4, int64_t(a.d) * 4,
                             int64_t(reinterpret_cast<uintptr_t>(a.q)), int64_t(reinterpret_cast<uintptr_t>(a.k))};
   const bool vec = common_vec_bytes(align, 5) == 16;

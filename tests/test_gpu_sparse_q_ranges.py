@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from cacheblend_vllm import _native
 from cacheblend_vllm import selection as S
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +68,32 @@ def test_f32_unaligned_views():
     _, want = S.sparse_q_full_scores(q.to(DEV), k.to(DEV), None, pos.to(DEV), 0.125, want_full=True)
     _, got = S.sparse_q_full_scores(off(q), off(k), None, pos.to(DEV), 0.125, want_full=True)
     assert torch.equal(got, want)
+
+
+def test_f32_more_keys_than_the_column_pass_holds():
+    # 2^31 (key, KV head) pairs: only the first keys are seen, and read
+    nk, hkv, seen, lib = (1 << 30) - 1, 2, 100, _native.load()
+    g = torch.Generator().manual_seed(1)
+    k = torch.empty(nk, hkv, 1, device=DEV)
+    first = torch.randn(seen + 1, hkv, 1, generator=g)
+    k[:seen + 1] = first.to(DEV)
+    q, pos = torch.randn(1, hkv, 1, generator=g), torch.tensor([seen])
+    index = torch.tensor([*range(seen + 2), 1 << 29, nk - 1], device=DEV)
+    out = torch.empty(index.numel(), device=DEV)
+    ws = torch.empty(lib.cbk_sparse_q_workspace_bytes(1, nk, hkv, hkv), dtype=torch.uint8, device=DEV)
+    dq, dp = q.to(DEV), pos.to(DEV)
+    rc = lib.cbk_sparse_q_scores(
+        dq.data_ptr(), hkv, None, 1, dp.data_ptr(), k.data_ptr(), hkv, nk, hkv, hkv, 1, 1.0,
+        _native.DTYPE_CODES[torch.float32], 0, index.data_ptr(), index.numel(), out.data_ptr(), None,
+        ws.data_ptr(), ws.numel(), _native.stream_handle(DEV))
+    _native.check(rc, "sparse_q_scores")
+    want, _ = _f64(q, first, torch.tensor([0]), pos, 1.0)
+    got = out.cpu().numpy()
+    del k, ws
+    torch.cuda.empty_cache()
+    # one product, ~100 exponentials and their sum, each within a few 2^-24
+    assert np.all(np.abs(got[:seen + 1] - want) <= 300 * 2.0 ** -24 * want)
+    assert np.all(got[seen + 1:] == 0)
 
 
 # few rows over many keys: up to 64 key ranges (more than the merge's batch of
