@@ -367,7 +367,10 @@ int cbk_blend_assemble_chunks(const cbk_kv_desc* kv, const int64_t* slots_dev,
  * npu_fused_infer_attention_score or the einsum path) with the causal mask
  * q_pos < k_pos evaluated in the kernel. bf16/f16: head_dim 64 or 128,
  * 16-byte aligned pointers and row strides, K/V row strides < 2^24
- * elements; float32: head_dim <= 128.
+ * elements; float32: head_dim <= 128. A visible key whose logit is -inf (a
+ * float16 product below -65504 rounds to it) has no weight; a row with no
+ * other is zero, NaN in float32. float32 keys and values past a row's position
+ * may hold anything.
  */
 int cbk_blend_attention(const void* q_dev, int64_t q_row_stride_elems, const int64_t* q_pos_dev, int64_t nq,
                         const void* k_dev, int64_t k_row_stride_elems, const void* v_dev,
@@ -391,10 +394,11 @@ int cbk_blend_attention_ws(const void* q_dev, int64_t q_row_stride_elems, const 
                            float scale, int32_t dtype, void* out_dev, int64_t out_row_stride_elems,
                            void* workspace_dev, size_t workspace_bytes, cbk_stream_t stream);
 
-/* Workspace bytes cbk_sparse_q_scores needs: row statistics, a record per
- * 16-query tile, per-KV-head partial column sums and a dense copy of the
- * query rows (sized for head_dim 128): about nq * hq * 264 + nk * hkv * 4
- * bytes. */
+/* Workspace bytes cbk_sparse_q_scores needs. Per (query, head), queries padded
+ * to a multiple of 64: 264 bytes (row statistics, a dense copy of the query row
+ * sized for head_dim 128) and 8 per key range (8 ranges; up to 64 while they
+ * all take at most 16 MB). Per (key, KV head): 16 (the partial column sums of 4
+ * query ranges). Per 16 queries: a record of 128. */
 size_t cbk_sparse_q_workspace_bytes(int64_t nq, int64_t nk, int64_t hq, int64_t hkv);
 
 /*

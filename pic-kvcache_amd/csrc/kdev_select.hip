@@ -1587,12 +1587,10 @@ int launch_select(const float* scores, const uint8_t* gap, const uint8_t* forced
 
 constexpr int kDilTile = 1024;
 
-__global__ __launch_bounds__(256) void dilate_kernel(const uint8_t* gap, uint32_t n, int32_t r,
-                                                      uint8_t* out) {
-  extern __shared__ uint32_t win[];  // kDilTile + 2r prefix counts
-  __shared__ uint32_t scan[8];
-  const uint32_t tile0 = blockIdx.x * kDilTile;
-  const uint32_t W = kDilTile + 2 * r;
+// win[w] = the flags set among tokens tile0 - r .. tile0 - r + w (those outside
+// [0, n) are not), for w < W, by a block of 256. Ends with a barrier.
+__device__ __forceinline__ void window_counts(const uint8_t* gap, uint32_t n, uint32_t tile0, int32_t r, uint32_t W,
+                                              uint32_t* win, uint32_t* scan) {
   const uint32_t per = (W + 255) / 256;
   const uint32_t beg = threadIdx.x * per;
   const uint32_t end = min(W, beg + per);
@@ -1606,6 +1604,14 @@ __global__ __launch_bounds__(256) void dilate_kernel(const uint8_t* gap, uint32_
   const uint32_t excl = block_exclusive_scan<256>(local, scan, &total);
   for (uint32_t w = beg; w < end; ++w) win[w] += excl;
   __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void dilate_kernel(const uint8_t* gap, uint32_t n, int32_t r,
+                                                      uint8_t* out) {
+  extern __shared__ uint32_t win[];  // kDilTile + 2r prefix counts
+  __shared__ uint32_t scan[8];
+  const uint32_t tile0 = blockIdx.x * kDilTile;
+  window_counts(gap, n, tile0, r, kDilTile + 2 * r, win, scan);
   for (uint32_t t = threadIdx.x; t < kDilTile; t += 256) {
     const uint32_t i = tile0 + t;
     if (i >= n) break;
@@ -1650,22 +1656,7 @@ __global__ __launch_bounds__(256) void sparse_q_masks_kernel(const uint8_t* gap,
   __shared__ uint32_t scan[8];
   const uint32_t tile0 = blockIdx.x * kRowTile;
   const uint32_t i0 = tile0 + threadIdx.x * kRowItems;
-  if (r > 0) {
-    const uint32_t W = kRowTile + 2 * r;
-    const uint32_t per = (W + 255) / 256;
-    const uint32_t beg = threadIdx.x * per;
-    const uint32_t end = min(W, beg + per);
-    uint32_t local = 0;
-    for (uint32_t w = beg; w < end; ++w) {
-      const int64_t g = int64_t(tile0) - r + w;
-      local += (g >= 0 && g < int64_t(n) && gap[g]) ? 1u : 0u;
-      win[w] = local;
-    }
-    uint32_t total;
-    const uint32_t excl = block_exclusive_scan<256>(local, scan, &total);
-    for (uint32_t w = beg; w < end; ++w) win[w] += excl;
-    __syncthreads();
-  }
+  if (r > 0) window_counts(gap, n, tile0, r, kRowTile + 2 * r, win, scan);
   const uint32_t bits = i0 < n ? flag_bits8(gap, i0, n) : 0u;
   uint64_t out = 0;
 #pragma unroll

@@ -27,7 +27,7 @@ struct SqArgs {
   float2* chunk_stats;    // [row_chunks][hq][nq_pad] (m2, l) of each key range, row_chunks > 1
   uint32_t row_chunks;    // key ranges per (query tile, kv head) in rowstats
   int32_t* tiles;         // [nq_pad / 16][32]: the 16 query positions (-1 past nq), min, max, unused
-  float* partial;         // [hkv][nk]
+  float* partial;         // [col_splits][hkv][nk] column sums of each query range
   uint16_t* qdense;       // [hkv][nq_pad / 16][groups][16][D]: query rows in colsum's unit order
   uint32_t nq_pad;
   uint32_t col_splits;    // query-unit ranges per (key block, kv head) in colsum
