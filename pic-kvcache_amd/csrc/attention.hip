@@ -297,10 +297,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   const uint32_t S = a.parts.splits;
   const uint32_t kvh = __builtin_amdgcn_readfirstlane(blockIdx.x % a.hkv);
   const uint32_t rest = __builtin_amdgcn_readfirstlane(blockIdx.x / a.hkv);
-  const uint32_t split = __builtin_amdgcn_readfirstlane(rest % S);
+  const uint32_t rank = S == 1 ? rest : __builtin_amdgcn_readfirstlane(rest / S);
+  const uint32_t split = rest - rank * S;
   const uint32_t nrows = a.nq * a.group;
   const uint32_t ntiles = (nrows + kRows - 1) / kRows;
-  const uint32_t tile = __builtin_amdgcn_readfirstlane(ntiles - 1 - rest / S);
+  const uint32_t tile = __builtin_amdgcn_readfirstlane(ntiles - 1 - rank);
   const uint32_t r_wave = tile * kRows + wave * 16 * RT;
 
   // this lane's rows (one per row tile): (query, head) and their Q fragments
@@ -344,8 +345,12 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(D =
   // the range)
   const uint32_t tile_blocks =
       gmax < 0 ? 0u : uint32_t(min((gmax + kKeyBlock) / kKeyBlock, (int32_t(a.nk) + kKeyBlock - 1) / kKeyBlock));
-  const int32_t b_lo = __builtin_amdgcn_readfirstlane(int32_t(uint64_t(tile_blocks) * split / S));
-  const int32_t nblocks = __builtin_amdgcn_readfirstlane(int32_t(uint64_t(tile_blocks) * (split + 1) / S)) - b_lo;
+  // (below 2^26 blocks and 2^5 ranges: 32 bits; a 64-bit division costs 0.2 us)
+  int32_t b_lo = 0, nblocks = __builtin_amdgcn_readfirstlane(int32_t(tile_blocks));
+  if (S > 1) {
+    b_lo = __builtin_amdgcn_readfirstlane(int32_t(tile_blocks * split / S));
+    nblocks = __builtin_amdgcn_readfirstlane(int32_t(tile_blocks * (split + 1) / S)) - b_lo;
+  }
   const int32_t key0 = b_lo * kKeyBlock;
   const int32_t nk = int32_t(a.nk) - key0;
   const uint16_t* const k_range = a.k + int64_t(key0) * a.k_stride;
