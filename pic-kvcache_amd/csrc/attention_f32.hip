@@ -68,6 +68,10 @@ __device__ void attend_row(const AttnF32Args& a, uint32_t qi, uint32_t h, int32_
     o0 = o0 * alpha + p * (lane < a.d ? vr[lane] : 0.f);
     o1 = o1 * alpha + p * (lane + 64 < a.d ? vr[lane + 64] : 0.f);
     m = mn;
+    if (l != l) {  // NaN from here on in every lane (uniform): a bad key that many rows see early
+      o0 = o1 = l;
+      return;
+    }
   }
 }
 
