@@ -143,7 +143,8 @@ def test_f32_keys_that_are_not_finite_reach_the_rows_that_see_them_only(nq, d, b
 # logits around the type's lowest and largest value, which times log2 e are
 # infinite, and an infinite value whose key's probability is 0
 @pytest.mark.parametrize("ranges", [False, True])
-@pytest.mark.parametrize("logits", [(-3e38, -3e38), (3e38, 3e38), (-3e38, -2.5e38), (-3e38, 1.0), (-1.5e38, -2.9e38)])
+@pytest.mark.parametrize("logits", [(-3e38, -3e38), (3e38, 3e38), (-3e38, -2.5e38), (-3e38, 1.0), (-1.5e38, -2.9e38),
+                                    (-np.inf, 1.0), (-np.inf, -np.inf)])
 def test_f32_logits_of_any_size(logits, ranges):
     nq, nk, hq, hkv, d = 20, 900, 2, 1, 64
     q, k, v, _ = _inputs(nq, nk, hq, hkv, d, seed=5)
@@ -155,6 +156,9 @@ def test_f32_logits_of_any_size(logits, ranges):
     want, mass, size = _f64(q, k, v, pos, 1.0)
     got, whole = _attend_in_guards(*(t.to(DEV) for t in (q, k, v, pos)), 1.0, ranges)
     assert whole
+    if max(logits) == -np.inf:  # no key has a weight: NaN, as the softmax is
+        assert bool(torch.isnan(got).all())
+        return
     assert np.all(np.abs(got.numpy() - want) <= _f32_bound(mass, 0.0, d, nk, 1.0))
     if logits == (-3e38, 1.0):
         # seen by all rows, at a probability of 0 of those that see a key past the first ranges
